@@ -1,0 +1,119 @@
+"""Dense fp32 attention on split operands (``csrc/dense_split.hip``) against
+float64: sizes around its tiles and chunks, and the rows that leave its fast
+path (a late large score, values too far apart for two parts, values that are
+not finite).
+
+Tolerance: the split kernel keeps q and k to 2^-24 and v and the weights to
+2^-22 of each value; the exponent's rounding, |c s| 2^-24 for scores up to
+about 2^5, is the largest term: 2^-19 of a weight, 4e-6 normwise with the sum
+of the others.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+RTOL = 4e-6
+
+
+def batch(N, least=3):
+    """The smallest batch of N agents that takes the split kernel."""
+    return max(least, -(-1024 // -(-N // 32)))
+
+
+def heads(B, N, d, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    return [torch.randn(B, N, d, generator=g).cuda() for _ in range(3)]
+
+
+def exact(q, k, v):
+    q, k, v = q.double(), k.double(), v.double()
+    s = torch.matmul(q, k.transpose(1, 2).contiguous()) / q.shape[-1] ** 0.5
+    s.diagonal(dim1=1, dim2=2).fill_(float("-inf"))
+    return torch.matmul(torch.softmax(s, -1), v), torch.logsumexp(s, -1)
+
+
+def check(out, ref):
+    """Every output row against its own largest entry."""
+    err = (out.double() - ref).abs().amax(-1) / ref.abs().amax(-1)
+    assert float(err.max()) <= RTOL * 4, float(err.max())
+    assert float((out.double() - ref).norm() / ref.norm()) <= RTOL
+
+
+@pytest.mark.parametrize("d", [16, 32, 64])
+@pytest.mark.parametrize("N", [33, 65, 95, 96, 97, 127, 129, 160, 255, 256, 257, 289, 513, 1000])
+def test_sizes(N, d):
+    from tarmac.kernels import dense_attention_forward_stats
+    q, k, v = heads(batch(N), N, d, seed=N + d)
+    out, stats = dense_attention_forward_stats(q, k, v)
+    ref, lse = exact(q, k, v)
+    check(out, ref)
+    got = stats[:, 0].double() * np.log(2.0)
+    assert float((got - lse).abs().max()) <= 2e-5
+
+
+@pytest.mark.parametrize("d", [16, 32, 64])
+def test_more_items_than_workgroups(d):
+    """Workgroups that take several rows in turn, with V scales that differ."""
+    from tarmac.kernels import fused_dense_attention
+    q, k, v = heads(1100, 70, d)
+    v *= torch.exp2(torch.arange(1100, device="cuda").remainder(41) - 20.0).view(-1, 1, 1)
+    check(fused_dense_attention(q, k, v), exact(q, k, v)[0])
+
+
+@pytest.mark.parametrize("d", [16, 32, 64])
+@pytest.mark.parametrize("log2_gap", [8, 14, 40, 90, 120, 200])
+def test_late_large_scores(d, log2_gap):
+    """A key beyond the first tile scores up to 2^gap times the others: the
+    offset is raised, or the row runs again, in steps along the row."""
+    from tarmac.kernels import fused_dense_attention
+    q, k, v = heads(batch(300), 300, d, seed=log2_gap)
+    c = np.log2(np.e) / d ** 0.5
+    for at, part in ((70, 0.3), (140, 0.6), (290, 1.0)):
+        k[1, at] = q[1, 17] / q[1, 17].norm() ** 2 * (part * log2_gap / c)
+    check(fused_dense_attention(q, k, v), exact(q, k, v)[0])
+
+
+@pytest.mark.parametrize("d", [16, 32, 64])
+@pytest.mark.parametrize("scale", [1e-30, 1e-12, 1e12, 1e30])
+def test_value_scales(d, scale):
+    from tarmac.kernels import fused_dense_attention
+    q, k, v = heads(batch(200), 200, d)
+    v = v * scale
+    check(fused_dense_attention(q, k, v), exact(q, k, v)[0])
+
+
+@pytest.mark.parametrize("d", [16, 32, 64])
+def test_values_far_apart(d):
+    """One agent's value row is 1e25 times the others' and no one attends to
+    it; another batch row grows along its keys from chunk to chunk."""
+    from tarmac.kernels import fused_dense_attention
+    q, k, v = heads(batch(400), 400, d)
+    q[0, :, 0], k[0, :, 0] = 40.0, 1.0
+    k[0, 150] = 0.0
+    k[0, 150, 0] = -40.0 * d ** 0.5
+    v[0, 150] = 1e25
+    v[1] *= torch.exp2(torch.arange(400, device="cuda") / 25.0).view(-1, 1)
+    q[2, 5] = 0.0  # a query of equal scores
+    ref = exact(q, k, v)[0]
+    out = fused_dense_attention(q, k, v)
+    check(out[0, torch.arange(400) != 150][None], ref[0, torch.arange(400) != 150][None])
+    check(out[1:], ref[1:])
+
+
+def test_not_finite_stays_in_its_row():
+    from tarmac.kernels import fused_dense_attention
+    q, k, v = heads(batch(130), 130, 16)
+    v[1, 3, 2] = float("inf")
+    k[2, 7, 1] = float("nan")
+    out = fused_dense_attention(q, k, v)
+    ref = exact(q, k, v)[0]
+    check(out[3:], ref[3:])
+    check(out[:1], ref[:1])
+    keep = torch.arange(16) != 2
+    check(out[1][:, keep][None], ref[1][:, keep][None])
+    assert not bool(torch.isfinite(out[1, 4:, 2]).any())
+    others = torch.arange(130) != 7
+    assert bool(torch.isnan(out[2, others]).all())

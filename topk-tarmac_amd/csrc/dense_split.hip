@@ -1,0 +1,381 @@
+// Dense attention in fp32 on 16-bit matrix instructions (d = 16, 32, 64),
+// every fp32 operand split into parts, sums in fp32.
+//
+// Why: the fp32 MFMA runs at 64 FLOP a cycle and SIMD and blocks the VALU
+// meanwhile; the bf16 / fp16 one at 1024, and its 32 x 32 form beside the
+// VALU (24 half-rate VALU operations and one 32x32x16: 46 ns against 43 for
+// the VALU alone and 14 for the MFMA; two 16x16x32 in its place: 53).
+//
+//   S^T = K Q^T      K and q in three bf16 parts (24 significand bits, fp32's
+//       exponent range): the six products of 2^-16 or more.
+//   O^T += V^T P^T   V and P in two fp16 parts (22 bits): all products at
+//       d = 16, where one 32-row operand holds V's hi and lo parts, three of
+//       four above. Two parts halve P's split (2 VALU a score, not 4) and the
+//       products. The parts' range is seen to, so that no value loses bits:
+//       V is scaled by a power of two that puts the row's largest magnitude
+//       below 2^15, its lo part by 2^11 more (its sums are kept apart), and a
+//       row with a nonzero element below 2^-29 of the largest takes the fp32
+//       form; P = 2^(c s - off) is kept below 2^15 with a sum of 2^5 or more.
+//   Error against 64 bits, N(0, 1) inputs: about half the fp32 MFMA kernel's.
+//   The A operand V^T comes from row-major rows by the transposing LDS read.
+//
+// Exponents: off is fixed per query before the first block, the maximum over
+// the row's first 32 keys less 5. Chains start at -off, so the product returns
+// the exponent itself. A block whose terms reach 2^15 raises off by a power of
+// two first (rare: 7 nats above the first keys). A wave with a query that still
+// ends out of range, or with values that are not finite, runs its queries again
+// on fp32 MFMA with a running maximum, from global memory.
+//
+// Loads: a workgroup's items (query blocks) and their key chunks form one
+// stream. The next chunk's K and V are loaded into registers while the current
+// one is computed on.
+//
+// Measured against the fp32 MFMA kernel (us): B=1024 N=256 d=16 44.1 -> 29.8,
+// d=32 84.2 -> 49.2, d=64 152 -> 99; B=256 N=1024 d=16 165 -> 106; B=36 N=1000
+// d=64 151 -> 80. Bound by VALU issue at d = 16 (about 100 VALU and 10 MFMA per
+// 32 x 32 tile and wave, the VALU busy three quarters of the time), by the
+// matrix core at d = 64 (36 MFMA a tile).
+#include <algorithm>
+
+#include "dense.hpp"
+#include "parts.hpp"
+
+namespace tarmac {
+
+constexpr float kSplitWindow = 5.f;      // log2 of the first tile's largest term
+constexpr float kSplitBlockMax = 0x1p15f;
+constexpr float kLoScale = 0x1p11f;
+
+template <int D>
+struct DenseSplit {
+  static constexpr int G = D / 16;          // 16-channel groups of a score product
+  static constexpr int NB = D > 32 ? D / 32 : 1;  // 32-row blocks of O^T
+  static constexpr int LDK = 3 * D + 8;     // halves per staged K row: hi, mid, lo
+  static constexpr int LDV = 2 * D + 8;     // halves per staged V row: hi, lo
+  static constexpr int VPR = D / 4;         // 16-byte vectors per fp32 row
+  static constexpr int KC = 2048 / D;       // most keys per chunk
+  static constexpr size_t lds_bytes(int kc) {
+    return static_cast<size_t>(kc) * (LDK + LDV) * 2 + 16;
+  }
+};
+
+// The rerun: 16 queries of a wave on fp32 MFMA, K and V^T fragments straight
+// from global memory, the running maximum raised per 16-key tile; writes the
+// outputs.
+template <int D>
+__device__ __forceinline__ void dense_online_global(const float* __restrict__ Qb,
+                                                    const float* __restrict__ Kb,
+                                                    const float* __restrict__ Vb,
+                                                    float* __restrict__ Ob, float* lse, int N,
+                                                    int q0, int lane, float c) {
+  using F = Frag<float, D>;
+  constexpr int NH = D / 16;
+  const int col = lane & 15, grp = lane >> 4, qi = q0 + col;
+  F frag;
+  frag.load_q(Qb + static_cast<size_t>(min(qi, N - 1)) * D, grp, c);
+  f32x4 acc[NH];
+#pragma unroll
+  for (int h = 0; h < NH; ++h) acc[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float off = -INFINITY, l = 0.f;
+#pragma unroll 1
+  for (int k0 = 0; k0 < N; k0 += 16) {
+    const typename F::KF kf = F::load_k(Kb + static_cast<size_t>(min(k0 + col, N - 1)) * D, grp);
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < F::NI; ++i) s = frag.step(kf, i, s);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int key = k0 + 4 * grp + r;
+      if (key >= N || key == qi) s[r] = -INFINITY;
+    }
+    const float m = query_max4(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])));
+    if (m > off + kDenseLag) {
+      const float alpha = fast_exp2(off - m);
+      l *= alpha;
+#pragma unroll
+      for (int h = 0; h < NH; ++h) acc[h] *= alpha;
+      off = m;
+    }
+    const float neg = off == -INFINITY ? 0.f : -off;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      s[r] = fast_exp2(s[r] + neg);
+      l += s[r];
+    }
+#pragma unroll
+    for (int h = 0; h < NH; ++h)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int row = k0 + 4 * grp + u;
+        const float x = row < N ? Vb[static_cast<size_t>(row) * D + 16 * h + col] : 0.f;
+        acc[h] = mfma_f32_16x16x4(x, s[u], acc[h]);
+      }
+  }
+  l = add_xor32(add_xor16(l));
+  if (qi >= N) return;
+  if (lse != nullptr && grp == 0) lse[qi] = off + log2f(l);
+  const float inv = __builtin_amdgcn_rcpf(l);
+#pragma unroll
+  for (int h = 0; h < NH; ++h) {
+    float o[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = acc[h][r] * inv;
+    st_f32<4>(Ob + static_cast<size_t>(qi) * D + 16 * h + 4 * grp, o);
+  }
+}
+
+// U: 16-byte vectors of K, and of V, per thread and chunk.
+template <int D, int U>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 4)))
+dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
+                   const float* __restrict__ V, float* __restrict__ O, float* __restrict__ lse,
+                   int N, int n_qblk, int kc, float scale, int nblocks) {
+  using DS = DenseSplit<D>;
+  constexpr int G = DS::G, NB = DS::NB, LDK = DS::LDK, LDV = DS::LDV, VPR = DS::VPR;
+  constexpr bool STACKED = D == 16;  // hi and lo rows of V^T in one operand
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  bf16* const Ks = reinterpret_cast<bf16*>(smem_raw);
+  bf16* const Vs = Ks + static_cast<size_t>(kc) * LDK;
+  // per parity of the item: the row's largest |v| (bits), and whether some
+  // element is too small beside it for two parts
+  uint32_t* const vmax = reinterpret_cast<uint32_t*>(Vs + static_cast<size_t>(kc) * LDV);
+  uint32_t* const tiny = vmax + 2;
+
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nw = blockDim.x >> 6, bd = blockDim.x;
+  const int col = lane & 31, half = lane >> 5;
+  const int self = col - 4 * half;  // tile_row of the self pair in a diagonal tile
+  const bf16* const Kl = Ks + col * LDK + 8 * half;
+  // this lane's 8-byte piece of the transposing reads: row 4 half + (l % 16) / 4
+  const bf16* const Vl = Vs + (4 * half + ((lane & 15) >> 2)) * LDV +
+                         ((lane >> 4) & 1) * (STACKED ? D : 16) + 4 * (lane & 3);
+
+  f32x4 xk[U], xv[U];  // the next chunk's vectors of this thread
+  auto load_chunk = [&](int b, int c0) {
+    const size_t base = (static_cast<size_t>(b) * N + c0) * D;
+    const int avail = min(kc, N - c0) * VPR;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int v = threadIdx.x + u * bd;
+      xk[u] = xv[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (v < avail) {
+        xk[u] = *reinterpret_cast<const f32x4*>(Kx + base + 4 * v);
+        xv[u] = *reinterpret_cast<const f32x4*>(V + base + 4 * v);
+      }
+    }
+  };
+  // item numbers are uniform; kept in SGPRs, so row bases are too
+  const int grid = gridDim.x;
+  int blk = __builtin_amdgcn_readfirstlane(xcd_logical_block(blockIdx.x, grid));
+  if (blk >= nblocks) return;
+  load_chunk(blk / n_qblk, 0);
+  if (threadIdx.x < 4) vmax[threadIdx.x] = 0u;
+  lds_barrier();
+  for (int par = 0; blk < nblocks; blk = __builtin_amdgcn_readfirstlane(blk + grid), par ^= 1) {
+    const int b = __builtin_amdgcn_readfirstlane(blk / n_qblk), qblk = blk - b * n_qblk;
+    const int q0 = __builtin_amdgcn_readfirstlane((qblk * nw + wave) * 32);
+    const size_t boff = static_cast<size_t>(b) * N * D;
+    RowParts<D> q;
+    q.load(Q + boff + static_cast<size_t>(min(q0 + col, N - 1)) * D, half, scale * kLog2e);
+    f32x16 acc[NB], accl[STACKED ? 1 : NB];  // stacked: elements 8..15 are the lo part's
+#pragma unroll
+    for (int n = 0; n < NB; ++n) acc[n] = f32x16{};
+    if constexpr (!STACKED)
+#pragma unroll
+      for (int n = 0; n < NB; ++n) accl[n] = f32x16{};
+    float off = 0.f, l = 0.f, vs = 0.f;  // vs: the scale of V so far (0: none yet)
+    for (int c0 = 0; c0 < N; c0 += kc) {
+      const int cn = min(kc, N - c0), kend = c0 + cn;
+      // V's largest magnitude so far in the row
+      float mx = 0.f;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(xv[u][0]), fabsf(xv[u][1])),
+                             fmaxf(fabsf(xv[u][2]), fabsf(xv[u][3]))));
+      mx = row16_reduce(mx, [](float a, float y) { return fmaxf(a, y); });
+      mx = query_max4(mx);
+      if (lane == 0) atomicMax(vmax + par, __float_as_uint(mx));
+      lds_barrier();  // also: the last chunk has been computed on
+      const uint32_t ef = max(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(vmax[par])) >> 23, 27u);
+      const float vs_new = __uint_as_float((268u - ef) << 23);  // 2^(14 - exponent)
+      if (c0 == 0 && threadIdx.x == 0) vmax[par ^ 1] = tiny[par ^ 1] = 0u;
+      uint32_t low = 0xffffffffu;  // the smallest nonzero |v|, scaled, less one ulp
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int v = threadIdx.x + u * bd, row = v / VPR, cv = v - row * VPR;
+        if (row < kc) {
+          store_parts3<D>(Ks + row * LDK + 4 * cv, xk[u]);
+          f16x2 vh[2], vl[2];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float x = xv[u][e] * vs_new;
+            low = min(low, (__float_as_uint(x) & 0x7fffffffu) - 1u);
+            vh[e / 2][e % 2] = static_cast<_Float16>(x);
+            vl[e / 2][e % 2] =
+                static_cast<_Float16>((x - static_cast<float>(vh[e / 2][e % 2])) * kLoScale);
+          }
+          bf16* vd = Vs + row * LDV + 4 * cv;
+          *reinterpret_cast<uint2*>(vd) = __builtin_bit_cast(uint2, vh);
+          *reinterpret_cast<uint2*>(vd + D) = __builtin_bit_cast(uint2, vl);
+        }
+      }
+      if (__any(low < 0x38800000u - 1u) && lane == 0) tiny[par] = 1u;  // below 2^-14
+      if (kend < N) load_chunk(b, kend);
+      else if (blk + grid < nblocks) load_chunk(__builtin_amdgcn_readfirstlane((blk + grid) / n_qblk), 0);
+      lds_barrier();
+      if (q0 < N) {
+        if (vs != vs_new) {  // uniform: the first chunk, or one with a larger |v|
+          const float r = vs == 0.f ? 0.f : vs_new * __uint_as_float((254u << 23) - __float_as_uint(vs));
+          vs = vs_new;
+#pragma unroll
+          for (int n = 0; n < NB; ++n) acc[n] *= r;
+          if constexpr (!STACKED)
+#pragma unroll
+            for (int n = 0; n < NB; ++n) accl[n] *= r;
+        }
+        for (int kb = 0; kb < cn; kb += 32) {
+          f32x16 s;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) s[i] = -off;
+          s = tile_dot<D>(q, Kl + kb * LDK, s);
+          const int kabs = c0 + kb;
+          if (kabs == q0) {  // the diagonal tile
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+              if (tile_row(i) == self) s[i] = -INFINITY;
+          }
+          if (kabs + 32 > kend) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+              if (tile_row(i) >= kend - kabs - 4 * half) s[i] = -INFINITY;
+          }
+          if (kabs == 0) {  // the first tile: off from its maximum
+            float m = -INFINITY;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) m = fmaxf(m, s[i]);
+            m = max_xor32(m);
+            off = m == -INFINITY ? 0.f : m - kSplitWindow;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[i] -= off;
+          }
+          float e[16], lb = 0.f;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) e[i] = fast_exp2(s[i]);
+#pragma unroll
+          for (int i = 0; i < 16; ++i) lb += e[i];
+          if (__any(!(lb < kSplitBlockMax))) {  // rare: raise off where a term is out of range
+            float m = 0.f;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) m = fmaxf(m, e[i]);
+            m = max_xor32(m);
+            // 2^-x with x = exponent(m) - 5 where m >= 2^11, else 1
+            const uint32_t em = __float_as_uint(m) >> 23;
+            const float r = em >= 138u && em < 255u ? __uint_as_float((259u - em) << 23) : 1.f;
+            off -= __builtin_amdgcn_logf(r);
+            l *= r;
+            lb *= r;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) e[i] *= r;
+#pragma unroll
+            for (int n = 0; n < NB; ++n) acc[n] *= r;
+            if constexpr (!STACKED)
+#pragma unroll
+              for (int n = 0; n < NB; ++n) accl[n] *= r;
+          }
+          l += lb;
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            uint32_t ph[4], pl[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) split2_pair(e[8 * t + 2 * i], e[8 * t + 2 * i + 1], ph[i], pl[i]);
+            const f16x8 p_hi = __builtin_bit_cast(f16x8, ph), p_lo = __builtin_bit_cast(f16x8, pl);
+            const bf16* vp = Vl + (kb + 16 * t) * LDV;
+#pragma unroll
+            for (int n = 0; n < NB; ++n) {
+              const f16x8 vh = __builtin_bit_cast(f16x8, load_t<LDV>(vp + 32 * n));
+              acc[n] = mfma_f16_32(vh, p_lo, acc[n]);
+              acc[n] = mfma_f16_32(vh, p_hi, acc[n]);
+              if constexpr (!STACKED) 
+                accl[n] = mfma_f16_32(__builtin_bit_cast(f16x8, load_t<LDV>(vp + D + 32 * n)), p_hi, accl[n]);
+            }
+          }
+        }
+      }
+    }
+    if (q0 < N) {
+      l = add_xor32(l);
+      // the sum of 2^4 or more, and every channel finite
+      float o[NB][16], a = 0.f;
+#pragma unroll
+      for (int n = 0; n < NB; ++n)
+#pragma unroll
+        for (int i = 0; i < (STACKED ? 8 : 16); ++i) {
+          o[n][i] = fmaf(STACKED ? acc[n][(i + 8) % 16] : accl[STACKED ? 0 : n][i], 1.f / kLoScale, acc[n][i]);
+          a = fmaf(0.f, o[n][i], a);
+        }
+      const bool fine = l >= 16.f && a == 0.f && tiny[par] == 0u;
+      float* const lse_row = lse == nullptr ? nullptr : lse + static_cast<size_t>(b) * 2 * N;
+      if (__any(!fine)) {
+#pragma unroll 1
+        for (int t = 0; t < 2; ++t)
+          if (q0 + 16 * t < N)
+            dense_online_global<D>(Q + boff, Kx + boff, V + boff, O + boff, lse_row, N, q0 + 16 * t,
+                                   lane, scale * kLog2e);
+      } else if (q0 + col < N) {
+        if (lse_row != nullptr && half == 0) lse_row[q0 + col] = off + log2f(l);
+        // 1 / vs is a power of two
+        const float inv = __builtin_amdgcn_rcpf(l) * __uint_as_float((254u << 23) - __float_as_uint(vs));
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+          for (int i = 0; i < (STACKED ? 8 : 16); i += 4) {
+            float w[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) w[r] = o[n][i + r] * inv;
+            st_f32<4>(O + boff + static_cast<size_t>(q0 + col) * D + 32 * n + 2 * i + 4 * half, w);
+          }
+      }
+    }
+  }
+}
+
+template <int D, int U>
+static hipError_t launch_dense_split_u(const DenseArgs& a, int nw, int n_qblk) {
+  using DS = DenseSplit<D>;
+  // equal chunks of what the threads can hold, at most KC keys
+  int kc = std::min(DS::KC, U * 64 * nw / DS::VPR / 32 * 32);
+  const int nch = (a.N + kc - 1) / kc;
+  kc = std::min(kc, ((a.N + nch - 1) / nch + 31) / 32 * 32);
+  const int nblocks = a.B * n_qblk;
+  // workgroups stay for as many items as it takes: sixteen waves per CU
+  const int grid = std::min(nblocks, kCUs * (16 / nw));
+  hipLaunchKernelGGL((dense_split_kernel<D, U>), dim3(grid), dim3(64 * nw), DS::lds_bytes(kc),
+                     static_cast<hipStream_t>(a.stream), static_cast<const float*>(a.q),
+                     static_cast<const float*>(a.k), static_cast<const float*>(a.v),
+                     static_cast<float*>(a.out), a.stats, a.N, n_qblk, kc, a.scale, nblocks);
+  return hipGetLastError();
+}
+
+template <int D>
+static hipError_t launch_dense_split(const DenseArgs& a) {
+  const int waves = (a.N + 31) / 32;
+  int nw = 8;
+  while (nw > 4 && a.B * ((waves + nw - 1) / nw) < 2 * kCUs) nw /= 2;  // more CUs at work
+  const int n_qblk = (waves + nw - 1) / nw;
+  nw = (waves + n_qblk - 1) / n_qblk;
+  if (nw == 8) return launch_dense_split_u<D, 1>(a, nw, n_qblk);
+  // d = 64: two vectors of three waves are less than a 32-key block
+  if (nw >= 4 || D < 64) return launch_dense_split_u<D, 2>(a, nw, n_qblk);
+  return launch_dense_split_u<D, 4>(a, nw, n_qblk);
+}
+
+hipError_t run_dense_split(const DenseArgs& a) {
+  switch (a.d) {
+    case 16: return launch_dense_split<16>(a);
+    case 32: return launch_dense_split<32>(a);
+    case 64: return launch_dense_split<64>(a);
+  }
+  return hipErrorInvalidValue;
+}
+
+}  // namespace tarmac

@@ -145,6 +145,7 @@ int set_query_tiles_mode(int mode);  // returns the previous mode
 bool one_query_tile(int B, int N);   // the launch shape under the current mode
 int query_tiles_mode();              // kTilesAuto, kTilesOne or kTilesTwo
 hipError_t run_dense(const DenseArgs& a);
+hipError_t run_dense_split(const DenseArgs& a);  // fp32, d = 16, 32, 64: dense_split.hip
 hipError_t run_fixedset(const FixedsetArgs& a);
 hipError_t run_morton_window(const MortonArgs& a);
 hipError_t run_zorder(const ZorderArgs& a);
