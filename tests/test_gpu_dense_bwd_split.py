@@ -1,0 +1,86 @@
+"""Dense backward on split operands (``csrc/backward_split.hip``) against
+float64 autograd: sizes around its tiles, chunks and launch shapes, gradients
+of any scale, and inputs that are not finite.
+
+Tolerance: 1e-5 of the largest entry, the bar of the fp32 gradient tests.
+"""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5
+
+
+def batch(N, least=3):
+    """The smallest batch of N agents that takes the split kernels."""
+    return max(least, -(-1024 // -(-N // 32)))
+
+
+def case(B, N, d, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    return [torch.randn(B, N, d, generator=g).cuda() for _ in range(4)]
+
+
+def exact(q, k, v, dout):
+    a = [t.double().requires_grad_(True) for t in (q, k, v)]
+    s = torch.matmul(a[0], a[1].transpose(1, 2).contiguous()) / q.shape[-1] ** 0.5
+    eye = torch.eye(q.shape[1], dtype=torch.bool, device=q.device)
+    out = torch.matmul(torch.softmax(s.masked_fill(eye, float("-inf")), -1), a[2])
+    return torch.autograd.grad(out, a, dout.double())
+
+
+def grads(q, k, v, dout, with_stats=True):
+    from tarmac.kernels import dense_attention_backward, dense_attention_forward_stats
+    out, stats = dense_attention_forward_stats(q, k, v)
+    return dense_attention_backward(q, k, v, out, dout, stats if with_stats else None)
+
+
+def check(got, ref):
+    for g, r in zip(got, ref):
+        assert float((g.double() - r).abs().max() / r.abs().max()) <= TOL
+        assert float((g.double() - r).norm() / r.norm()) <= 2e-6
+
+
+@pytest.mark.parametrize("d", [16, 32, 64])
+@pytest.mark.parametrize("N", [33, 65, 96, 97, 128, 129, 160, 255, 256, 257, 300, 513])
+def test_sizes(N, d):
+    x = case(batch(N), N, d, seed=N + d)
+    check(grads(*x), exact(*x))
+
+
+@pytest.mark.parametrize("d", [16, 32, 64])
+def test_launch_shapes(d):
+    """Eight-wave workgroups over full rows, more items than workgroups, and
+    the logsumexp formed by the backward itself."""
+    x = case(520 if d == 16 else 300, 256, d)
+    ref = exact(*x)
+    check(grads(*x), ref)
+    check(grads(*x, with_stats=False), ref)
+    x = case(1100, 70, d)
+    check(grads(*x), exact(*x))
+
+
+@pytest.mark.parametrize("d", [16, 32, 64])
+@pytest.mark.parametrize("scale", [1e-33, 1e-20, 1e20])
+def test_gradient_scales(d, scale):
+    q, k, v, dout = case(batch(150), 150, d)
+    check(grads(q, k, v, dout * scale), exact(q, k, v, dout * scale))
+
+
+@pytest.mark.parametrize("d", [16, 64])
+def test_zero_and_not_finite_rows(d):
+    q, k, v, dout = case(batch(100), 100, d)
+    dout[0] = 0.0
+    dout[1, 5, 3] = float("inf")
+    dq, dk, dv = grads(q, k, v, dout)
+    for g in (dq, dk, dv):
+        assert bool((g[0] == 0).all())
+    ref = exact(q, k, v, dout)
+    check([g[2:] for g in (dq, dk, dv)], [r[2:] for r in ref])
+    # the other queries of that row, and the other channels of its dv
+    others = torch.arange(100) != 5
+    check([dq[1:2, others]], [ref[0][1:2, others]])
+    keep = torch.arange(d) != 3
+    check([dv[1:2, :, keep]], [ref[2][1:2, :, keep]])

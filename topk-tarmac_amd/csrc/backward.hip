@@ -1029,11 +1029,24 @@ static hipError_t launch_dense_bwd(const DenseBwdArgs& a) {
   hipStream_t st = static_cast<hipStream_t>(a.stream);
   const size_t lds_q = dq_lds_bytes<D>((kc + BQ - 1) / BQ * BQ);
   const size_t lds_kv = dkv_lds_bytes<D>((qc + BQ - 1) / BQ * BQ);
-  hipLaunchKernelGGL((dense_bwd_dq_kernel<D, T>), dim3(nblocks), dim3(64 * nw), lds_q, st, a.q,
-                     a.k, a.v, a.out, a.dout, a.dq, a.stats, a.stats_ready, a.N, nblk, kc, a.scale,
-                     nblocks);
-  hipError_t e = hipGetLastError();
+  // split operands once the batch gives every SIMD a wave of 32 rows (B=128
+  // N=256 d=16: 30.5 -> 23 us) on rows of more than two 32-row tiles, at d = 32
+  // more than one (B=512 N=40 d=32: 24.1 -> 19.3; B=1024 N=40 d=16 18.9 against
+  // 19.2, B=512 N=64 d=64 43.2 against 44.1). Pass 1 needs the forward's
+  // logsumexp; without it the fp32 pass forms it.
+  const bool split = (D == 16 || D == 32 || D == 64) && a.N > (D == 32 ? 32 : 64) &&
+      static_cast<long>(a.B) * ((a.N + 31) / 32) >= 4L * kCUs;
+  hipError_t e;
+  if (split && a.stats_ready) {
+    e = run_dense_bwd_split(a, false);
+  } else {
+    hipLaunchKernelGGL((dense_bwd_dq_kernel<D, T>), dim3(nblocks), dim3(64 * nw), lds_q, st, a.q,
+                       a.k, a.v, a.out, a.dout, a.dq, a.stats, a.stats_ready, a.N, nblk, kc, a.scale,
+                       nblocks);
+    e = hipGetLastError();
+  }
   if (e != hipSuccess) return e;
+  if (split) return run_dense_bwd_split(a, true);
   hipLaunchKernelGGL((dense_bwd_dkv_kernel<D, T>), dim3(nblocks), dim3(64 * nw), lds_kv, st, a.q,
                      a.k, a.v, a.dout, a.stats, a.dk, a.dv, a.N, nblk, qc, a.scale, nblocks);
   return hipGetLastError();

@@ -20,8 +20,7 @@
 //   The A operand V^T comes from row-major rows by the transposing LDS read.
 //
 // Exponents: off is fixed per query before the first block, the maximum over
-// the row's first 32 keys less 5. Chains start at -off, so the product returns
-// the exponent itself. A block whose terms reach 2^15 raises off by a power of
+// the row's first 32 keys less 5. A block whose terms reach 2^15 raises off by a power of
 // two first (rare: 7 nats above the first keys). A wave with a query that still
 // ends out of range, or with values that are not finite, runs its queries again
 // on fp32 MFMA with a running maximum, from global memory.
@@ -48,7 +47,6 @@ constexpr float kLoScale = 0x1p11f;
 
 template <int D>
 struct DenseSplit {
-  static constexpr int G = D / 16;          // 16-channel groups of a score product
   static constexpr int NB = D > 32 ? D / 32 : 1;  // 32-row blocks of O^T
   static constexpr int LDK = 3 * D + 8;     // halves per staged K row: hi, mid, lo
   static constexpr int LDV = 2 * D + 8;     // halves per staged V row: hi, lo
@@ -131,7 +129,7 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
                    const float* __restrict__ V, float* __restrict__ O, float* __restrict__ lse,
                    int N, int n_qblk, int kc, float scale, int nblocks) {
   using DS = DenseSplit<D>;
-  constexpr int G = DS::G, NB = DS::NB, LDK = DS::LDK, LDV = DS::LDV, VPR = DS::VPR;
+  constexpr int NB = DS::NB, LDK = DS::LDK, LDV = DS::LDV, VPR = DS::VPR;
   constexpr bool STACKED = D == 16;  // hi and lo rows of V^T in one operand
   extern __shared__ __align__(16) unsigned char smem_raw[];
   bf16* const Ks = reinterpret_cast<bf16*>(smem_raw);

@@ -104,22 +104,35 @@ struct RowParts {
 };
 
 // s + (32 staged rows) . (the columns' rows): rows at R (lane l: row l % 32 of
-// the tile plus 8 (l / 32) channels), stored as hi[D] mid[D] lo[D]; the small
-// products first.
+// the tile plus 8 (l / 32) channels), stored as hi[D] mid[D] lo[D]. A bf16 MFMA
+// cuts what it adds at the accumulator's last place, so the products of the
+// parts go in from the smallest up, over all channel groups before the next
+// larger ones, and a chain starts at 0 rather than at a large offset: only the
+// D / 16 products of the hi parts are rounded at the sum's own magnitude.
 template <int D>
 __device__ __forceinline__ f32x16 tile_dot(const RowParts<D>& q, const bf16* R, f32x16 s) {
+  constexpr int G = D / 16;
+  // d = 64 reads the rows' hi and mid parts again for the larger products:
+  // kept, they would take 32 registers that the kernels do not have
+  auto again = [&]() {
+    if constexpr (D > 32) asm volatile("" : "+v"(R) : : "memory");
+  };
+  auto part = [&](int p, int g) { return *reinterpret_cast<const bf16x8*>(R + p * D + 16 * g); };
 #pragma unroll
-  for (int g = 0; g < D / 16; ++g) {
-    const bf16x8 h = *reinterpret_cast<const bf16x8*>(R + 16 * g);
-    const bf16x8 m = *reinterpret_cast<const bf16x8*>(R + D + 16 * g);
-    const bf16x8 l = *reinterpret_cast<const bf16x8*>(R + 2 * D + 16 * g);
-    s = mfma_bf16_32(l, q.hi[g], s);
-    s = mfma_bf16_32(h, q.lo[g], s);
-    s = mfma_bf16_32(m, q.mid[g], s);
-    s = mfma_bf16_32(m, q.hi[g], s);
-    s = mfma_bf16_32(h, q.mid[g], s);
-    s = mfma_bf16_32(h, q.hi[g], s);
+  for (int g = 0; g < G; ++g) {
+    s = mfma_bf16_32(part(2, g), q.hi[g], s);
+    s = mfma_bf16_32(part(0, g), q.lo[g], s);
+    s = mfma_bf16_32(part(1, g), q.mid[g], s);
   }
+  again();
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    s = mfma_bf16_32(part(1, g), q.hi[g], s);
+    s = mfma_bf16_32(part(0, g), q.mid[g], s);
+  }
+  again();
+#pragma unroll
+  for (int g = 0; g < G; ++g) s = mfma_bf16_32(part(0, g), q.hi[g], s);
   return s;
 }
 

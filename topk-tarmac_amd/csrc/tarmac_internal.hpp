@@ -154,6 +154,9 @@ hipError_t run_mfma_bf16_probe(const void* a, const void* b, float* out, int T, 
                                int shape, void* stream);
 hipError_t run_fixedset_bwd(const FixedsetBwdArgs& a);
 hipError_t run_dense_bwd(const DenseBwdArgs& a);
+// fp32, d = 16, 32, 64, more than 32 rows: one pass of backward_split.hip (pass 1
+// takes the forward's logsumexp and writes dO.O; pass 2 reads both)
+hipError_t run_dense_bwd_split(const DenseBwdArgs& a, bool pass2);
 // Library-held device workspace (one per GPU, kScratchBytes): the current
 // device's address of it, looked up on the first call on that device.
 constexpr size_t kScratchBytes = size_t(8) << 20;
