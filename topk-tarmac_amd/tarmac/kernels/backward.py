@@ -80,7 +80,7 @@ def fixedset_attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tenso
     dv = torch.empty_like(v)
     if B == 0:  # an empty batch: nothing to launch
         return dq, dk, dv
-    with torch.cuda.device(q.device):
+    with _launch.on_device_of(q):
         rc = _lib.LIB.tarmac_fixedset_bwd(
             _launch.ptr(q), _launch.ptr(k), _launch.ptr(v), _launch.ptr(dout), _launch.ptr(idx),
             _lib.IDX_I64 if idx.dtype == torch.int64 else _lib.IDX_I32, idx.shape[-1],
@@ -103,7 +103,7 @@ def dense_attention_forward_stats(q: torch.Tensor, k: torch.Tensor, v: torch.Ten
     stats = torch.empty(B, 2, N, device=q.device, dtype=torch.float32)
     if B == 0:
         return out, stats
-    with torch.cuda.device(q.device):
+    with _launch.on_device_of(q):
         _lib.check(_lib.LIB.tarmac_dense_fwd_stats(
             _launch.ptr(q), _launch.ptr(k), _launch.ptr(v), _launch.ptr(out), _launch.ptr(stats),
             B, N, d, _launch.stream(q)))
@@ -133,7 +133,7 @@ def dense_attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         stats = torch.empty(B, 2, N, device=q.device, dtype=torch.float32)
     if B == 0:
         return dq, dk, dv
-    with torch.cuda.device(q.device):
+    with _launch.on_device_of(q):
         rc = _lib.LIB.tarmac_dense_bwd(
             _launch.ptr(q), _launch.ptr(k), _launch.ptr(v), _launch.ptr(out), _launch.ptr(dout),
             _launch.ptr(dq), _launch.ptr(dk), _launch.ptr(dv), _launch.ptr(stats), int(ready),

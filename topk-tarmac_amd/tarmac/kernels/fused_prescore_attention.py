@@ -35,7 +35,7 @@ def fused_prescore_attention(q: torch.Tensor, k: torch.Tensor,
     out = torch.empty_like(q)
     if B == 0:  # an empty batch: nothing to launch
         return out
-    with torch.cuda.device(q.device):
+    with _launch.on_device_of(q):
         _lib.check(_lib.LIB.tarmac_fixedset_fwd(
             _launch.ptr(q), _launch.ptr(k), _launch.ptr(v), _launch.ptr(idx), code,
             idx.shape[-1], _launch.ptr(out), B, N, d, _launch.dtype_code(q), _launch.stream(q)))

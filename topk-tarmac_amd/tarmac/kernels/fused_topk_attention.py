@@ -47,7 +47,7 @@ def topk_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, topk: int,
     idx = torch.empty(B, N, kk, device=q.device, dtype=torch.int32) if return_indices else None
     if B == 0:  # an empty batch: nothing to launch
         return (out, idx) if return_indices else out
-    with torch.cuda.device(q.device):
+    with _launch.on_device_of(q):
         if key_chunk is None:
             rc = _lib.LIB.tarmac_topk_fused_fwd(
                 _launch.ptr(q), _launch.ptr(k), _launch.ptr(v), _launch.ptr(out),
@@ -116,7 +116,7 @@ def topk_variant_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, to
     idx = torch.empty(B, N, kk, device=q.device, dtype=torch.int32) if return_indices else None
     if B == 0:
         return (out, idx) if return_indices else out
-    with torch.cuda.device(q.device):
+    with _launch.on_device_of(q):
         rc = _lib.LIB.tarmac_topk_variant_fwd(
             _launch.ptr(q), _launch.ptr(k), _launch.ptr(v), _launch.ptr(out), _launch.ptr(idx),
             B, N, d, kk, int(variant), int(bisect), _launch.dtype_code(q), _launch.stream(q))

@@ -47,7 +47,7 @@ def _morton_code(pos: torch.Tensor, bits: int = 10) -> torch.Tensor:
     codes = torch.empty(B, N, device=pos.device, dtype=torch.int64)
     if B == 0:  # an empty batch: nothing to launch
         return codes
-    with torch.cuda.device(pos.device):
+    with _launch.on_device_of(pos):
         _lib.check(_lib.LIB.tarmac_morton_window(
             _launch.ptr(pos), _launch.ptr(None), _lib.IDX_I64, _launch.ptr(codes),
             B, N, 1, int(bits), _launch.stream(pos)))
@@ -61,7 +61,7 @@ def select_morton_window(pos: torch.Tensor, k: int, bits: int = 10) -> torch.Ten
     idx = torch.empty(B, N, k, device=pos.device, dtype=torch.int64)
     if B == 0:
         return idx
-    with torch.cuda.device(pos.device):
+    with _launch.on_device_of(pos):
         _lib.check(_lib.LIB.tarmac_morton_window(
             _launch.ptr(pos), _launch.ptr(idx), _lib.IDX_I64, _launch.ptr(None),
             B, N, int(k), int(bits), _launch.stream(pos)))
@@ -74,7 +74,7 @@ def _knn(fn, pos: torch.Tensor, k: int) -> torch.Tensor:
     idx = torch.empty(B, N, int(k), device=pos.device, dtype=torch.int64)
     if B == 0:
         return idx
-    with torch.cuda.device(pos.device):
+    with _launch.on_device_of(pos):
         _lib.check(fn(_launch.ptr(pos), _launch.ptr(idx), _lib.IDX_I64, B, N, int(k),
                       _launch.stream(pos)))
     return idx
@@ -127,7 +127,7 @@ def zorder_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pos: tor
     idx = torch.empty(B, N, topk, device=q.device, dtype=torch.int32) if return_indices else None
     if B == 0:
         return (out, idx) if return_indices else out
-    with torch.cuda.device(q.device):
+    with _launch.on_device_of(q):
         _lib.check(_lib.LIB.tarmac_zorder_fwd(
             _launch.ptr(q), _launch.ptr(k), _launch.ptr(v), _launch.ptr(pos), _launch.ptr(out),
             _launch.ptr(idx), B, N, d, int(topk), int(bits), _launch.dtype_code(q),
