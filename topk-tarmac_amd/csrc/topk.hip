@@ -1162,17 +1162,23 @@ static TopkPath choose_path(const TopkArgs& a, int mode) {
   // again, 8.3 vs 9.0 at k = 1)
   if (a.topk <= 4 && a.N > 64 && (a.N <= 256 || a.B * a.N <= 16384) && one_query_tile(a.B, a.N))
     return kPathPacked;
-  // k = 1 at d = 32, 64 on rows of 512-1023 keys from B = 256: the filter
-  // (B=256 N=512/768 d=32: 44.1/88.1 vs 46.3/95.3 lists; d=64: 80.1/144.2 vs
-  // 83.2/167.0; at d = 16 the split-bf16 scores stay ahead, N=768: 40.4 vs
-  // 47.7)
-  if (filt && a.d >= 32 && a.topk == 1 && a.N >= 512 && a.N < 1024 && a.B >= 256)
+  // k = 1 at d = 64 on rows of 512-1023 keys from B = 256: the filter
+  // (B=256 N=512/768: 80.1/144.2 vs 83.2/167.0 lists, 83.5 on split-bf16 scores
+  // at N = 512; at d = 16 the split-bf16 scores stay ahead, N=768: 40.4 vs 47.7)
+  if (filt && a.d == 64 && a.topk == 1 && a.N >= 512 && a.N < 1024 && a.B >= 256)
     return kPathFilter;
-  // d = 64, k >= 3 on rows of 512 keys and more from B = 1024: the register
-  // lists (B=1024 N=512 k=3/4/6: 383.1/461.7/524.7 vs 408.1/514.2/580.0
-  // packed; B=2048 k=4: 862.8 vs 1016.0; at B = 256 packed stays ahead,
-  // 122.9 vs 124.0 at k = 4)
-  if (a.d == 64 && a.topk >= 3 && a.N >= 512 && a.B >= 1024) return kPathLists;
+  // split-bf16 scores at d = 32, 64 (six bf16 products take 6/16 of the fp32
+  // MFMA's time, but a split row is 1.4 times an fp32 row in LDS and costs its
+  // split): on long rows of batches that take two query tiles per wave. d = 32
+  // from N = 512 (B=256 N=512 k=1/2/4: 38.6/43.0/52.1 vs 43.0 filter, 51.0,
+  // 60.1 packed; B=1024 133.5/147.7/172.3 vs 151.2/179.9/213.0; N=1024
+  // 111/123/145 vs 122/154/199; below, B=1024 N=256 k=2 62.0 vs 53.9 lists).
+  // d = 64 at k >= 3 from N = 512 (B=256 k=4 108.3 vs 121.2 packed; B=1024
+  // k=4/8 446.9/620.1 vs 460.2/628.3 lists), at k = 1, 2 from N = 1024 (B=256
+  // 244.3/264.2 vs 277.4/303.8 lists; N=512 k=2 91.4 vs 90.2).
+  if (split && a.d >= 32 && a.N >= 512 && (a.d == 32 || a.topk >= 3 || a.N >= 1024) &&
+      !one_query_tile(a.B, a.N))
+    return kPathPackedSplit;
   // the lists at k <= 2 on rows of up to 128 keys up to B = 256 (B=256
   // N=128 k=1/2: 4.8/5.9 vs 5.4/6.1 on 32 x 32 tiles)
   if (a.topk <= 2 && a.N <= 128 && a.B <= 256) return kPathLists;
@@ -1186,7 +1192,7 @@ static TopkPath choose_path(const TopkArgs& a, int mode) {
   // vs 28.0 lists / 36.3 packed; B=4096 N=192 k=4: 111.2 vs 126.9), and at
   // N = 128 for k >= 3 once B >= 1024 (B=4096 N=128 k=3/4: 45.3/52.1 vs
   // 47.0/53.6 packed; k = 2 stays on the lists there, 39.4 vs 40.4)
-  if (split && (a.N >= 160 || (a.N >= 128 && a.B >= 1024 && a.topk >= 3))) return kPathPackedSplit;
+  if (split && a.d == 16 && (a.N >= 160 || (a.N >= 128 && a.B >= 1024 && a.topk >= 3))) return kPathPackedSplit;
   return (a.topk <= 2 || a.N <= 32) ? kPathLists : kPathPacked;
 }
 

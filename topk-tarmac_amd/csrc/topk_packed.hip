@@ -10,12 +10,15 @@ size_t packed_lds_bytes(int dtype, int d, int kc, bool split) {
   return 16 + static_cast<size_t>(kcb) * row;
 }
 
-bool packed_split_supported(int dtype, int d) { return dtype == kF32 && d == 16; }
+bool packed_split_supported(int dtype, int d) { return dtype == kF32 && (d == 16 || d == 32 || d == 64); }
 
 hipError_t run_topk_packed(const TopkArgs& a, bool split) {
   if (a.d == 128) return split ? hipErrorInvalidValue : run_topk_packed_d128(a);
   if (a.dtype == kF32) {
-    if (split) return a.d == 16 ? launch_packed<float, 16, true>(a) : hipErrorInvalidValue;
+    if (split) {
+      if (a.d == 32 || a.d == 64) return run_topk_packed_split_wide(a);
+      return a.d == 16 ? launch_packed<float, 16, true>(a) : hipErrorInvalidValue;
+    }
     switch (a.d) {
       case 8: return launch_packed<float, 8, false>(a);
       case 16: return launch_packed<float, 16, false>(a);
