@@ -1167,14 +1167,16 @@ static TopkPath choose_path(const TopkArgs& a, int mode) {
   // at N = 512; at d = 16 the split-bf16 scores stay ahead, N=768: 40.4 vs 47.7)
   if (filt && a.d == 64 && a.topk == 1 && a.N >= 512 && a.N < 1024 && a.B >= 256)
     return kPathFilter;
+  // d = 64, k >= 3 on rows of 512 keys and more from B = 1024: the register
+  // lists (B=1024 N=576 k=8: 800 vs 847 on split-bf16 scores, 860 packed)
+  if (a.d == 64 && a.topk >= 3 && a.N >= 512 && a.B >= 1024) return kPathLists;
   // split-bf16 scores at d = 32, 64 (six bf16 products take 6/16 of the fp32
   // MFMA's time, but a split row is 1.4 times an fp32 row in LDS and costs its
   // split): on long rows of batches that take two query tiles per wave. d = 32
   // from N = 512 (B=256 N=512 k=1/2/4: 38.6/43.0/52.1 vs 43.0 filter, 51.0,
   // 60.1 packed; B=1024 133.5/147.7/172.3 vs 151.2/179.9/213.0; N=1024
   // 111/123/145 vs 122/154/199; below, B=1024 N=256 k=2 62.0 vs 53.9 lists).
-  // d = 64 at k >= 3 from N = 512 (B=256 k=4 108.3 vs 121.2 packed; B=1024
-  // k=4/8 446.9/620.1 vs 460.2/628.3 lists), at k = 1, 2 from N = 1024 (B=256
+  // d = 64 at k >= 3 from N = 512 (B=256 k=4 108.3 vs 121.2 packed), at k = 1, 2 from N = 1024 (B=256
   // 244.3/264.2 vs 277.4/303.8 lists; N=512 k=2 91.4 vs 90.2).
   if (split && a.d >= 32 && a.N >= 512 && (a.d == 32 || a.topk >= 3 || a.N >= 1024) &&
       !one_query_tile(a.B, a.N))
