@@ -55,7 +55,9 @@ const char* tarmac_last_error(void);
  * Replaces src/kernels/fused_dense_attention.py:106-152 (fused_dense_attention)
  * and the composed dense paths scripts/bench_attention_core.py:74-82
  * (dense_unfused, dense_fused) / src/agents/mappo.py:174-190,361-372,418.
- * key_chunk: keys staged per LDS pass (0 = whole row when it fits).
+ * key_chunk: keys staged per LDS pass, a multiple of 16 (0 = the library's
+ * choice; N or more = the row, in chunks of the library's choice where the
+ * kernel that runs takes smaller ones).
  */
 int tarmac_dense_fwd(const void* q, const void* k, const void* v, void* out, int B, int N, int d,
                      int dtype, int key_chunk, void* stream);

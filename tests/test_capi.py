@@ -8,7 +8,10 @@ arguments with the documented codes before any HIP call is made.
 from __future__ import annotations
 
 import ctypes
+import os
 import re
+import subprocess
+import sys
 from pathlib import Path
 
 import pytest
@@ -95,6 +98,25 @@ def test_alignment_and_null_checks():
     rc = _lib.LIB.tarmac_topk_stream_fwd(_fake(), _fake(), _fake(), _fake(), None,
                                          2, 64, 16, 2, 0, 40, None)
     assert rc == 1 and "multiple of 16" in _lib.last_error()
+
+
+def test_dense_small_chunk_at_a_large_batch_returns():
+    """fp32 rows of 17 to 32 keys staged 16 at a time, from the batch on that
+    takes the split-operand kernel: the launcher's arithmetic holds (no
+    division by a chunk of zero keys) and the call returns a status. In a
+    process of its own, with every device hidden: no kernel can run."""
+    code = ("import ctypes\n"
+            "from tarmac import _lib\n"
+            "p = ctypes.c_void_p(256)\n"
+            "for d in (16, 32, 64):\n"
+            "    for N in (17, 24, 32, 33, 64):\n"
+            "        for chunk in (16, 32):\n"
+            "            rc = _lib.LIB.tarmac_dense_fwd(p, p, p, p, 1024, N, d, 0, chunk, None)\n"
+            "            assert rc == 3, (rc, d, N, chunk)\n")
+    env = dict(os.environ, HIP_VISIBLE_DEVICES="-1", ROCR_VISIBLE_DEVICES="-1",
+               PYTHONPATH=str(ROOT / "topk-tarmac_amd"))
+    run = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True)
+    assert run.returncode == 0, (run.returncode, run.stderr)
 
 
 def test_python_wrappers_refuse_cpu_tensors():

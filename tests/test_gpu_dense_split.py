@@ -55,6 +55,22 @@ def test_sizes(N, d):
 
 
 @pytest.mark.parametrize("d", [16, 32, 64])
+@pytest.mark.parametrize("N", [17, 24, 32, 33, 64, 96])
+def test_chunk_below_the_row(N, d):
+    """A caller's chunk is kept at every batch: the kernel that stages it gives
+    a row the same bits at B = 1024, past the line of the split kernel, as at
+    B = 2."""
+    from tarmac.kernels import fused_dense_attention
+    q, k, v = heads(1024, N, d, seed=N + d)
+    ref = exact(q, k, v)[0]
+    for chunk in (16, 32):
+        out = fused_dense_attention(q, k, v, block_kn=chunk)
+        check(out, ref)
+        if chunk < N:
+            assert torch.equal(out[:2], fused_dense_attention(q[:2], k[:2], v[:2], block_kn=chunk))
+
+
+@pytest.mark.parametrize("d", [16, 32, 64])
 def test_more_items_than_workgroups(d):
     """Workgroups that take several rows in turn, with V scales that differ."""
     from tarmac.kernels import fused_dense_attention

@@ -408,6 +408,7 @@ template <int D, int U, bool PASS2>
 hipError_t launch_pass(const DenseBwdArgs& a, int nw, int n_blk) {
   using BS = BwdSplit<D>;
   int kc = std::min(BS::KC, U * 64 * nw / BS::VPR / 32 * 32);
+  if (kc < 32) return hipErrorInvalidValue;  // fewer threads than a 32-row block takes
   const int nch = (a.N + kc - 1) / kc;
   kc = std::min(kc, ((a.N + nch - 1) / nch + 31) / 32 * 32);
   const int nblocks = a.B * n_blk;

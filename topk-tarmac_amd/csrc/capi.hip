@@ -143,6 +143,7 @@ int dense_common(const void* q, const void* k, const void* v, void* out, float* 
   if (tarmac::dense_lds_bytes(dtype, d, kc) > dense_lds_budget(d))
     return fail(TARMAC_ERR_UNSUPPORTED, "%s: key_chunk %d exceeds the LDS budget at d=%d", fn, kc, d);
   tarmac::DenseArgs a{q, k, v, out, B, N, d, dtype, kc, inv_sqrt(d), stream, stats};
+  a.chunk_given = key_chunk > 0;
   return hip_status(tarmac::run_dense(a), fn);
 }
 

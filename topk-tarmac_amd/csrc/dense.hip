@@ -411,9 +411,14 @@ static hipError_t launch_dense(const DenseArgs& a) {
     // on fp32 MFMA finish first (B=32: N=256 d=16 6.3 vs 9.5 us, d=32 9.2 vs
     // 14.0, N=512 d=64 30.6 vs 35.2; at the line B=128 N=256: 8.7 vs 8.5,
     // 14.7 vs 13.7, d=64 26.4 vs 19.9). The line follows the sizes alone, so
-    // the query-tiles override leaves outputs as they are.
+    // the query-tiles override leaves outputs as they are. A caller's chunk
+    // below the row is kept (the split kernel chooses its own chunks), and rows
+    // of one 32-query wave at d = 32 and 64 reach this line only with one (its
+    // workgroup of one wave could not stage 32 keys).
     if constexpr (D == 16 || D == 32 || D == 64)
-      if (static_cast<long>(a.B) * ((a.N + 31) / 32) >= 4L * kCUs) return run_dense_split(a);
+      if ((!a.chunk_given || a.key_chunk >= a.N) &&
+          static_cast<long>(a.B) * ((a.N + 31) / 32) >= 4L * kCUs)
+        return run_dense_split(a);
   }
   if (one_query_tile(a.B, a.N)) return launch_dense_q<T, D, 1>(a);
   if constexpr (sizeof(T) == 2 && D <= 32) {

@@ -342,6 +342,7 @@ static hipError_t launch_dense_split_u(const DenseArgs& a, int nw, int n_qblk) {
   using DS = DenseSplit<D>;
   // equal chunks of what the threads can hold, at most KC keys
   int kc = std::min(DS::KC, U * 64 * nw / DS::VPR / 32 * 32);
+  if (kc < 32) return hipErrorInvalidValue;  // fewer threads than a 32-key block takes
   const int nch = (a.N + kc - 1) / kc;
   kc = std::min(kc, ((a.N + nch - 1) / nch + 31) / 32 * 32);
   const int nblocks = a.B * n_qblk;

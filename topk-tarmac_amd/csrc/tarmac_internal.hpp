@@ -46,6 +46,7 @@ struct DenseArgs {
   float scale;
   void* stream;
   float* stats = nullptr;  // nullable: [B, 2, N] workspace, plane 0 gets the logsumexp
+  bool chunk_given = false;  // key_chunk is the caller's, not the library's choice
 };
 
 struct FixedsetArgs {
