@@ -232,10 +232,7 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
             for (int n = 0; n < NB; ++n) accl[n] *= r;
         }
         for (int kb = 0; kb < cn; kb += 32) {
-          f32x16 s;
-#pragma unroll
-          for (int i = 0; i < 16; ++i) s[i] = -off;
-          s = tile_dot<D>(q, Kl + kb * LDK, s);
+          f32x16 s = tile_dot<D>(q, Kl + kb * LDK, f32x16{});
           const int kabs = c0 + kb;
           if (kabs == q0) {  // the diagonal tile
 #pragma unroll
@@ -253,12 +250,10 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
             for (int i = 0; i < 16; ++i) m = fmaxf(m, s[i]);
             m = max_xor32(m);
             off = m == -INFINITY ? 0.f : m - kSplitWindow;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) s[i] -= off;
           }
           float e[16], lb = 0.f;
 #pragma unroll
-          for (int i = 0; i < 16; ++i) e[i] = fast_exp2(s[i]);
+          for (int i = 0; i < 16; ++i) e[i] = fast_exp2(s[i] - off);
 #pragma unroll
           for (int i = 0; i < 16; ++i) lb += e[i];
           if (__any(!(lb < kSplitBlockMax))) {  // rare: raise off where a term is out of range
@@ -320,7 +315,11 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
             dense_online_global<D>(Q + boff, Kx + boff, V + boff, O + boff, lse_row, N, q0 + 16 * t,
                                    lane, scale * kLog2e);
       } else if (q0 + col < N) {
-        if (lse_row != nullptr && half == 0) lse_row[q0 + col] = off + log2f(l);
+        // log2 of the sum by exponent and mantissa: the logarithm's own error
+        // is then at the last place of 1, not of log2 l (10 and more)
+        if (lse_row != nullptr && half == 0)
+          lse_row[q0 + col] = (off + static_cast<float>(__builtin_amdgcn_frexp_expf(l))) +
+                              log2f(__builtin_amdgcn_frexp_mantf(l));
         // 1 / vs is a power of two
         const float inv = __builtin_amdgcn_rcpf(l) * __uint_as_float((254u << 23) - __float_as_uint(vs));
 #pragma unroll
