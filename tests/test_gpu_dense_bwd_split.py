@@ -51,6 +51,17 @@ def test_sizes(N, d):
 
 
 @pytest.mark.parametrize("d", [16, 32, 64])
+@pytest.mark.parametrize("N,N1_error", [(100, 3.0e-7), (256, 4.1e-7)])
+def test_no_further_from_float64_than_fp32_mfma(N, N1_error, d):
+    """N(0, 1) inputs: the normwise error of each gradient against that of the
+    fp32 MFMA kernels at d = 16 (the smallest of dq, dk, dv; d = 64 has four
+    times the products a score and 1.2 times the error)."""
+    x = case(batch(N), N, d, seed=1)
+    for g, r in zip(grads(*x), exact(*x)):
+        assert float((g.double() - r).norm() / r.norm()) <= N1_error * (1.2 if d == 64 else 1.0)
+
+
+@pytest.mark.parametrize("d", [16, 32, 64])
 def test_launch_shapes(d):
     """Eight-wave workgroups over full rows, more items than workgroups, and
     the logsumexp formed by the backward itself."""

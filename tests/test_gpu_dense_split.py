@@ -80,6 +80,20 @@ def test_more_items_than_workgroups(d):
 
 
 @pytest.mark.parametrize("d", [16, 32, 64])
+@pytest.mark.parametrize("N", [100, 256, 1000])
+def test_logsumexp_is_not_one_sided(N, d):
+    """The mean error over all rows, which the backward would carry into every
+    gradient. An fp32 logsumexp of 2^2 to 2^3 rounds at 2^-23 of it without a
+    sign: its mean over B N rows is far below 1e-7, the bound here; sums of
+    2^10 rounded down at their own last place gave 3.4e-7."""
+    from tarmac.kernels import dense_attention_forward_stats
+    q, k, v = heads(batch(N), N, d, seed=N)
+    _, stats = dense_attention_forward_stats(q, k, v)
+    err = stats[:, 0].double() * np.log(2.0) - exact(q, k, v)[1]
+    assert abs(float(err.mean())) <= 1e-7
+
+
+@pytest.mark.parametrize("d", [16, 32, 64])
 @pytest.mark.parametrize("log2_gap", [8, 14, 40, 90, 120, 200])
 def test_late_large_scores(d, log2_gap):
     """A key beyond the first tile scores up to 2^gap times the others: the
