@@ -113,11 +113,16 @@ template <int D>
 __device__ __forceinline__ f32x16 tile_dot(const RowParts<D>& q, const bf16* R, f32x16 s) {
   constexpr int G = D / 16;
   // d = 64 reads the rows' hi and mid parts again for the larger products:
-  // kept, they would take 32 registers that the kernels do not have
+  // kept, they would take 32 registers that the kernels do not have. The
+  // opaque copy is of the LDS address (of a generic pointer it would make the
+  // reads flat ones, which wait for the global loads in flight).
+  using lds_t = const __attribute__((address_space(3))) bf16x8;
+  using lds_row = const __attribute__((address_space(3))) bf16;
+  lds_row* L = (lds_row*)R;
   auto again = [&]() {
-    if constexpr (D > 32) asm volatile("" : "+v"(R) : : "memory");
+    if constexpr (D > 32) asm volatile("" : "+v"(L));
   };
-  auto part = [&](int p, int g) { return *reinterpret_cast<const bf16x8*>(R + p * D + 16 * g); };
+  auto part = [&](int p, int g) { return *(lds_t*)(L + p * D + 16 * g); };
 #pragma unroll
   for (int g = 0; g < G; ++g) {
     s = mfma_bf16_32(part(2, g), q.hi[g], s);
