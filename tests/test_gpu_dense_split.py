@@ -133,6 +133,25 @@ def test_values_far_apart(d):
     check(out[1:], ref[1:])
 
 
+@pytest.mark.parametrize("d", [16, 32, 64])
+@pytest.mark.parametrize("log2_value", [6, 10, 14, 18])
+@pytest.mark.parametrize("log2_weight", [-9, -15, -20])
+def test_small_weights_of_large_values(d, log2_value, log2_weight):
+    """Each query attends to one agent; the others weigh 2^-9 to 2^-20 of it
+    and their values are 2^6 to 2^18 times as large, so the output is the sum
+    of small weights and has to keep their relative precision."""
+    from tarmac.kernels import fused_dense_attention
+    N = 256
+    q, k, v = heads(batch(N), N, d, seed=log2_value)
+    gap = -log2_weight * np.log(2.0) * d ** 0.5
+    q[1], k[1] = q[1] * 0.01, k[1] * 0.01
+    q[1, :, 0], k[1, :, 0] = 1.0, -gap
+    k[1, 77, 0] = 0.0  # the agent attended to
+    v[1] *= 2.0 ** log2_value
+    v[1, 77] *= 2.0 ** -log2_value
+    check(fused_dense_attention(q, k, v), exact(q, k, v)[0])
+
+
 def test_not_finite_stays_in_its_row():
     from tarmac.kernels import fused_dense_attention
     q, k, v = heads(batch(130), 130, 16)

@@ -297,16 +297,27 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
     }
     if (q0 < N) {
       l = add_xor32(l);
-      // the sum of 2^4 or more, and every channel finite
-      float o[NB][16], a = 0.f;
+      float a = 0.f, big = 0.f, small = INFINITY;
 #pragma unroll
       for (int n = 0; n < NB; ++n)
 #pragma unroll
         for (int i = 0; i < (STACKED ? 8 : 16); ++i) {
-          o[n][i] = fmaf(STACKED ? acc[n][(i + 8) % 16] : accl[STACKED ? 0 : n][i], 1.f / kLoScale, acc[n][i]);
-          a = fmaf(0.f, o[n][i], a);
+          acc[n][i] = fmaf(STACKED ? acc[n][(i + 8) % 16] : accl[STACKED ? 0 : n][i], 1.f / kLoScale, acc[n][i]);
+          a = fmaf(0.f, acc[n][i], a);
+          big = fmaxf(big, fabsf(acc[n][i]));
+          small = fminf(small, fabsf(acc[n][i]));
         }
-      const bool fine = l >= 16.f && a == 0.f && tiny[par] == 0u;
+      big = max_xor32(big);
+      // Whether the parts kept what fp32 keeps: the sum of 2^4 or more; every
+      // channel finite; the query's largest channel so large that N terms
+      // rounded at 2^-25 beside values below 2^15 stay below 2^-20 of it (a
+      // wave of sharp rows beside values 2^5 and more times theirs fails
+      // this); and, in a row with an element below 2^-14, every channel above
+      // 2^-14 of the sum.
+      const bool zeros = __builtin_amdgcn_readfirstlane(vmax[par]) == 0u;
+      const bool wide = __builtin_amdgcn_readfirstlane(tiny[par]) != 0u;
+      const float least = zeros ? 0.f : 1024.f * __builtin_amdgcn_sqrtf(static_cast<float>(N));
+      const bool fine = (l >= 16.f) & (a == 0.f) & (big >= least) & (small >= (wide ? l * 0x1p-14f : 0.f));
       float* const lse_row = lse == nullptr ? nullptr : lse + static_cast<size_t>(b) * 2 * N;
       if (__any(!fine)) {
 #pragma unroll 1
@@ -328,7 +339,7 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
           for (int i = 0; i < (STACKED ? 8 : 16); i += 4) {
             float w[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) w[r] = o[n][i + r] * inv;
+            for (int r = 0; r < 4; ++r) w[r] = acc[n][i + r] * inv;
             st_f32<4>(O + boff + static_cast<size_t>(q0 + col) * D + 32 * n + 2 * i + 4 * half, w);
           }
       }
