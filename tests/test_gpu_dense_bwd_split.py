@@ -80,6 +80,21 @@ def test_gradient_scales(d, scale):
     check(grads(q, k, v, dout * scale), exact(q, k, v, dout * scale))
 
 
+@pytest.mark.parametrize("d", [16, 32, 64])
+@pytest.mark.parametrize("scale", [1e-33, 1e-34])
+def test_small_gradients_beside_ordinary_ones(d, scale):
+    """Every other query's output gradient, and one of its channels for the
+    others, is far below its neighbours': each row of dq and each channel of dv
+    is held against its own size."""
+    q, k, v, dout = case(batch(150), 150, d)
+    dout[:, ::2] *= scale
+    dout[:, :, 5] = dout[:, :1, 5]
+    dq, dk, dv = grads(q, k, v, dout)
+    ref = exact(q, k, v, dout)
+    check([dq[:, ::2], dq[:, 1::2]], [ref[0][:, ::2], ref[0][:, 1::2]])
+    check([dv[:, :, 5:6], dv[:, :, :5]], [ref[2][:, :, 5:6], ref[2][:, :, :5]])
+
+
 @pytest.mark.parametrize("d", [16, 64])
 def test_zero_and_not_finite_rows(d):
     q, k, v, dout = case(batch(100), 100, d)

@@ -16,8 +16,8 @@
 //     tiles with rows and columns exchanged (lse and D come from LDS);
 //     dV^T += dO^T P, dK^T += Q^T dS.
 //
-// A wave whose outputs are not all finite, or all below 2^-70 (parts of the
-// terms would leave the normal range), runs again on fp32 MFMA from global
+// A wave with an output that is not finite, or nonzero and below 2^-80 (parts
+// of its terms may have left their range), runs again on fp32 MFMA from global
 // memory. One barrier a chunk: the next chunk is loaded into registers while
 // the current one is computed on, then split into the other LDS buffer.
 //
@@ -124,21 +124,23 @@ __device__ __forceinline__ void fold_halves(f32x16 (&acc)[BwdSplit<D>::NB]) {
 }
 constexpr int grad_elems(int D) { return D == 16 ? 8 : 16; }
 
-// Whether the fast path's result stands: finite, and zero or of a size whose
-// parts are normal numbers. mx collects |x|, nan the products 0 * x.
+// Whether a lane's part of a result stands: every element finite, and zero or
+// of 2^-80 or more. Parts keep a value to 2^-134, so an element loses bits of
+// fp32's 24 only below 2^-110 times the sum of the magnitudes beside its small
+// factors: 2^30, for instance 1024 rows of values up to 2^20.
+constexpr uint32_t kGradTiny = 0x17800000u;  // 2^-80
 template <int D>
-__device__ __forceinline__ void scan_grad(const f32x16 (&acc)[BwdSplit<D>::NB], float& mx, float& nan) {
+__device__ __forceinline__ bool grad_stands(const f32x16 (&acc)[BwdSplit<D>::NB]) {
+  float nan = 0.f;
+  uint32_t low = 0xffffffffu;  // bits of the smallest nonzero magnitude, less one
 #pragma unroll
   for (int n = 0; n < BwdSplit<D>::NB; ++n)
 #pragma unroll
     for (int i = 0; i < grad_elems(D); ++i) {
-      mx = fmaxf(mx, fabsf(acc[n][i]));
+      low = min(low, (__float_as_uint(acc[n][i]) & 0x7fffffffu) - 1u);
       nan = fmaf(0.f, acc[n][i], nan);
     }
-}
-__device__ __forceinline__ bool wave_stands(float mx, float nan) {
-  const bool any_normal = __any(mx >= 0x1p-70f), any_tiny = __any(mx > 0.f && mx < 0x1p-70f);
-  return !__any(!(nan == 0.f)) && (any_normal || !any_tiny);
+  return (nan == 0.f) & (low >= kGradTiny - 1u);
 }
 
 template <int D>
@@ -378,15 +380,12 @@ dense_bwd_split_kernel(const float* __restrict__ colA, const float* __restrict__
     }
     if (x0 < N) {
       fold_halves<D>(ga);
-      float mx = 0.f, nan = 0.f;
-      scan_grad<D>(ga, mx, nan);
-      bool stands = wave_stands(mx, nan);
+      bool stands = grad_stands<D>(ga);
       if constexpr (PASS2) {
         fold_halves<D>(gb);
-        mx = nan = 0.f;
-        scan_grad<D>(gb, mx, nan);
-        stands = wave_stands(mx, nan) && stands;
+        stands &= grad_stands<D>(gb);
       }
+      stands = __all(stands);
       if (stands) {
         if (x0 + col < N) {
           store_grad<D>(out_a + boff + static_cast<size_t>(xi) * D, ga, half, scale);
