@@ -74,6 +74,13 @@ def test_launch_shapes(d):
 
 
 @pytest.mark.parametrize("d", [16, 32, 64])
+def test_one_vector_a_thread(d):
+    """Workgroups of eight waves (from 512 rows on): one vector a thread."""
+    x = case(520, 250, d)
+    check(grads(*x), exact(*x))
+
+
+@pytest.mark.parametrize("d", [16, 32, 64])
 @pytest.mark.parametrize("scale", [1e-33, 1e-20, 1e20])
 def test_gradient_scales(d, scale):
     q, k, v, dout = case(batch(150), 150, d)

@@ -22,12 +22,19 @@
 // the current one is computed on, then split into the other LDS buffer.
 //
 // Measured, both passes, against the fp32 MFMA kernels (us): B=1024 N=256 d=16
-// 172 -> 127, d=32 296 -> 199; B=256 N=512 d=16 163 -> 119; B=300 N=200 d=64
-// 228 -> 141. Bound by the matrix core and the VALU about equally at d = 16 (20
-// and 28 MFMA of 33 cycles, 140 and 240 VALU per 32 x 32 tile), by the matrix
-// core above. Error against 64 bits at d = 16, N = 256: dq, dk, dv 4.5, 4.5,
-// 4.4e-7 (fp32 MFMA 4.7, 4.3, 4.1e-7); N = 512 4.6, 4.5, 4.5e-7 (5.7, 5.2,
-// 5.1e-7); d = 64 5.0, 5.0, 5.0e-7 (4.9, 4.9, 4.7e-7).
+// 174 -> 120, d=32 298 -> 194, d=64 741 -> 387; B=256 N=512 d=16 165 -> 109;
+// B=300 N=200 d=64 230 -> 113. Per 32 x 32 tile the passes take 20 and 28 MFMA
+// of 33 cycles at d = 16 and 48 and 72 at d = 64, 140 and 240 VALU. Error against
+// 64 bits at d = 16, N = 256: dq, dk, dv 3.3, 3.3, 3.2e-7 (fp32 MFMA 4.7, 4.4,
+// 4.1e-7); N = 512 3.5, 3.4, 3.3e-7 (5.7, 5.2, 5.1e-7); d = 64, N = 256 4.1, 4.1,
+// 4.0e-7 (5.2, 5.2, 4.9e-7).
+//
+// Registers: at d = 64 pass 2 keeps 96 for its columns' parts and 64 for two
+// accumulators of the 256 that two waves a SIMD leave, and uses no scratch. What
+// else would live across the loops is kept out of it: row offsets are scalars
+// (uniform_offset), and lane addresses outside the loops come from opaque copies
+// of the lane number (with them in registers it spilled 20 to 68, and both
+// passes took B=300 N=200 d=64 133 us).
 #include <algorithm>
 
 #include "parts.hpp"
@@ -252,24 +259,28 @@ dense_bwd_split_kernel(const float* __restrict__ colA, const float* __restrict__
   f32x4 xa[U], xb[U];
   float xs = 0.f, xd = 0.f;
   auto load_chunk = [&](int b, int c0) {
-    const size_t base = (static_cast<size_t>(b) * N + c0) * D;
+    // uniform bases, so a thread's address is a 32-bit offset
+    const size_t base = uniform_offset((static_cast<size_t>(b) * N + c0) * D);
+    const char* const Ab = reinterpret_cast<const char*>(A + base);
+    const char* const Bb = reinterpret_cast<const char*>(Bm + base);
     const int rows = min(kc, N - c0), avail = rows * VPR;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int v = threadIdx.x + u * bd;
       xa[u] = xb[u] = f32x4{0.f, 0.f, 0.f, 0.f};
       if (v < avail) {
-        xa[u] = *reinterpret_cast<const f32x4*>(A + base + 4 * v);
-        xb[u] = *reinterpret_cast<const f32x4*>(Bm + base + 4 * v);
+        xa[u] = *reinterpret_cast<const f32x4*>(Ab + static_cast<uint32_t>(v) * 16u);
+        xb[u] = *reinterpret_cast<const f32x4*>(Bb + static_cast<uint32_t>(v) * 16u);
       }
     }
     if constexpr (PASS2) {  // a chunk has at most as many rows as threads
-      xs = -INFINITY;       // rows past the end: p = 0
+      const float* const lse = stats + uniform_offset(static_cast<size_t>(b) * 2 * N + c0);
+      const float* const dsum = lse + N;
+      xs = INFINITY;  // rows past the end: p = 0
       xd = 0.f;
       if (static_cast<int>(threadIdx.x) < rows) {
-        const float* st = stats + static_cast<size_t>(b) * 2 * N + c0 + threadIdx.x;
-        xs = -st[0];
-        xd = -st[N];
+        xs = lse[threadIdx.x];
+        xd = dsum[threadIdx.x];
       }
     }
   };
@@ -284,27 +295,31 @@ dense_bwd_split_kernel(const float* __restrict__ colA, const float* __restrict__
   for (; blk < nblocks; blk = __builtin_amdgcn_readfirstlane(blk + grid)) {
     const int b = __builtin_amdgcn_readfirstlane(blk / n_blk), xblk = blk - b * n_blk;
     const int x0 = __builtin_amdgcn_readfirstlane((xblk * nw + wave) * 32);
-    const size_t boff = static_cast<size_t>(b) * N * D;
-    float* const st = stats + static_cast<size_t>(b) * 2 * N;
-    const int xi = min(x0 + col, N - 1);
+    const size_t boff = uniform_offset(static_cast<size_t>(b) * N * D);
+    float* const st = stats + uniform_offset(static_cast<size_t>(b) * 2 * N);
+    // opaque copies of the lane number, here and after the loops: addresses
+    // formed from them are not kept in registers across the loops
+    int pl = lane;
+    asm volatile("" : "+v"(pl));
+    const int xi = min(x0 + (pl & 31), N - 1);
     RowParts<D> pa, pb;
-    pa.load(colA + boff + static_cast<size_t>(xi) * D, half, scale * kLog2eF);
-    pb.load(colB + boff + static_cast<size_t>(xi) * D, half, 1.f);
+    pa.load(colA + boff + static_cast<size_t>(xi) * D, pl >> 5, scale * kLog2eF);
+    pb.load(colB + boff + static_cast<size_t>(xi) * D, pl >> 5, 1.f);
     float nl = 0.f, nd = 0.f;  // pass 1: -lse and -D of the lane's query
     if constexpr (!PASS2) {
       float dd = 0.f;
 #pragma unroll
       for (int g = 0; g < D / 16; ++g) {
         float o[8], d[8];
-        ld_f32<8>(o, O + boff + static_cast<size_t>(xi) * D + 16 * g + 8 * half);
-        ld_f32<8>(d, colB + boff + static_cast<size_t>(xi) * D + 16 * g + 8 * half);
+        ld_f32<8>(o, O + boff + static_cast<size_t>(xi) * D + 16 * g + 8 * (pl >> 5));
+        ld_f32<8>(d, colB + boff + static_cast<size_t>(xi) * D + 16 * g + 8 * (pl >> 5));
 #pragma unroll
         for (int e = 0; e < 8; ++e) dd = fmaf(d[e], o[e], dd);
       }
       dd = add_xor32(dd);
       nd = -dd;
       nl = -st[xi];
-      if (half == 0 && x0 + col < N) st[N + xi] = dd;
+      if (pl < 32 && x0 + pl < N) st[N + xi] = dd;
     }
     f32x16 ga[NB], gb[PASS2 ? NB : 1];
 #pragma unroll
@@ -327,8 +342,8 @@ dense_bwd_split_kernel(const float* __restrict__ colA, const float* __restrict__
       }
       if constexpr (PASS2)
         if (static_cast<int>(threadIdx.x) < kc) {
-          Ls[threadIdx.x] = xs;
-          Ls[kc + threadIdx.x] = xd;
+          Ls[threadIdx.x] = -xs;
+          Ls[kc + threadIdx.x] = -xd;
         }
       if (kend < N) load_chunk(b, kend);
       else if (blk + grid < nblocks) load_chunk(__builtin_amdgcn_readfirstlane((blk + grid) / n_blk), 0);
@@ -386,18 +401,21 @@ dense_bwd_split_kernel(const float* __restrict__ colA, const float* __restrict__
         stands &= grad_stands<D>(gb);
       }
       stands = __all(stands);
+      int el = lane;
+      asm volatile("" : "+v"(el));
+      const int ecol = el & 31, exi = min(x0 + ecol, N - 1);
       if (stands) {
-        if (x0 + col < N) {
-          store_grad<D>(out_a + boff + static_cast<size_t>(xi) * D, ga, half, scale);
-          if constexpr (PASS2) store_grad<D>(out_b + boff + static_cast<size_t>(xi) * D, gb, half, 1.f);
+        if (x0 + ecol < N) {
+          store_grad<D>(out_a + boff + static_cast<size_t>(exi) * D, ga, el >> 5, scale);
+          if constexpr (PASS2) store_grad<D>(out_b + boff + static_cast<size_t>(exi) * D, gb, el >> 5, 1.f);
         }
       } else {
 #pragma unroll 1
         for (int t = 0; t < 2; ++t)
           if (x0 + 16 * t < N)
-            bwd_rerun<D, PASS2>(colA + boff, colB + boff, A + boff, Bm + boff, -__shfl(nl, 16 * t + (lane & 15)),
-                                -__shfl(nd, 16 * t + (lane & 15)), st, st + N, out_a + boff,
-                                PASS2 ? out_b + boff : nullptr, N, x0 + 16 * t, lane, scale);
+            bwd_rerun<D, PASS2>(colA + boff, colB + boff, A + boff, Bm + boff, -__shfl(nl, 16 * t + (el & 15)),
+                                -__shfl(nd, 16 * t + (el & 15)), st, st + N, out_a + boff,
+                                PASS2 ? out_b + boff : nullptr, N, x0 + 16 * t, el, scale);
       }
     }
   }
@@ -432,9 +450,12 @@ hipError_t launch_pass_d(const DenseBwdArgs& a) {
   while (nw > 4 && a.B * ((waves + nw - 1) / nw) < 2 * kCUs) nw /= 2;  // more CUs at work
   const int n_blk = (waves + nw - 1) / nw;
   nw = (waves + n_blk - 1) / n_blk;
+  // d = 64: two vectors a thread of fewer than four waves are less than a 32-row
+  // block, so rows of three waves have a fourth that only stages (four vectors
+  // a thread instead spilled 35 registers in pass 2)
+  if (D == 64) nw = std::max(nw, 4);
   if (nw == 8 || (D == 16 && PASS2 && nw == 4)) return launch_pass<D, 1, PASS2>(a, nw, n_blk);
-  if (nw >= 4 || D < 64) return launch_pass<D, 2, PASS2>(a, nw, n_blk);
-  return launch_pass<D, 4, PASS2>(a, nw, n_blk);
+  return launch_pass<D, 2, PASS2>(a, nw, n_blk);
 }
 
 }  // namespace

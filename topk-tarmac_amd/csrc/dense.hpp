@@ -1,7 +1,7 @@
-// The block loop of the dense attention kernels: scores, self and chunk-end
-// masks, exponents, row sums and the P.V product over one staged key chunk,
-// for operands in their own type (fp32 or bf16 MFMA). Shared by dense.hip and
-// by the split-operand kernel, which runs it on rows its own path cannot take.
+// The block loop of dense_kernel (dense.hip): scores, self and chunk-end masks,
+// exponents, row sums and the P.V product over one staged key chunk, for
+// operands in their own type (fp32 or bf16 MFMA). The split-operand kernel
+// (dense_split.hip) takes its constants and query_max4 from here.
 #pragma once
 
 #include "frag.hpp"

@@ -10,30 +10,36 @@
 //       exponent range): the six products of 2^-16 or more.
 //   O^T += V^T P^T   V and P in two fp16 parts (22 bits): all products at
 //       d = 16, where one 32-row operand holds V's hi and lo parts, three of
-//       four above. Two parts halve P's split (2 VALU a score, not 4) and the
-//       products. The parts' range is seen to, so that no value loses bits:
-//       V is scaled by a power of two that puts the row's largest magnitude
-//       below 2^15, its lo part by 2^11 more (its sums are kept apart), and a
-//       row with a nonzero element below 2^-29 of the largest takes the fp32
-//       form; P = 2^(c s - off) is kept below 2^15 with a sum of 2^5 or more.
-//   Error against 64 bits, N(0, 1) inputs: about half the fp32 MFMA kernel's.
+//       four above. Three bf16 parts of each (24 bits, no range to see to) cost
+//       21% at d = 16 and gave the same error. V is scaled by a power of two that
+//       puts the row's largest magnitude below 2^15, its lo part by 2^11 more
+//       (its sums are kept apart); P = 2^(c s - off) is kept below 2^15 with a
+//       sum of 2^4 or more.
+//   Error against 64 bits, N(0, 1) inputs, N = 256: 2.1, 2.1, 2.2e-7 at d = 16,
+//   32, 64 (fp32 MFMA: 6.2, 10.4, 4.0e-7); logsumexp 3e-8 off on average (5e-8).
 //   The A operand V^T comes from row-major rows by the transposing LDS read.
 //
 // Exponents: off is fixed per query before the first block, the maximum over
-// the row's first 32 keys less 5. A block whose terms reach 2^15 raises off by a power of
-// two first (rare: 7 nats above the first keys). A wave with a query that still
-// ends out of range, or with values that are not finite, runs its queries again
-// on fp32 MFMA with a running maximum, from global memory.
+// the row's first 32 keys less 5. A block whose terms reach 2^15 raises off by a
+// power of two first (rare: 7 nats above the first keys). Score chains start
+// at 0 and off is subtracted after: a chain that starts at off is cut at off's
+// magnitude in every product, which the backward sees at scores of 2^5 and more.
+//
+// The result decides whether the parts kept what fp32 keeps: P is held to
+// 2^-25 where it is below 2^-3, scaled V to 2^-36 below 2^-14. A wave with a
+// query whose sum is out of range, whose values are not finite, whose largest
+// channel is small beside what such rounding adds up to, or that has a channel
+// of the size of the smallest parts in a row that holds such elements, runs
+// its queries again on fp32 MFMA with a running maximum, from global memory.
 //
 // Loads: a workgroup's items (query blocks) and their key chunks form one
 // stream. The next chunk's K and V are loaded into registers while the current
 // one is computed on.
 //
-// Measured against the fp32 MFMA kernel (us): B=1024 N=256 d=16 44.1 -> 29.8,
-// d=32 84.2 -> 49.2, d=64 152 -> 99; B=256 N=1024 d=16 165 -> 106; B=36 N=1000
-// d=64 151 -> 80. Bound by VALU issue at d = 16 (about 100 VALU and 10 MFMA per
-// 32 x 32 tile and wave, the VALU busy three quarters of the time), by the
-// matrix core at d = 64 (36 MFMA a tile).
+// Measured against the fp32 MFMA kernel (us): B=1024 N=256 d=16 45.0 -> 31.8,
+// d=32 85.5 -> 47.6, d=64 153 -> 102; B=256 N=1024 d=16 166 -> 100; B=36 N=1000
+// d=64 152 -> 82. About 100 VALU and 10 MFMA per 32 x 32 tile and wave at d = 16,
+// 36 MFMA at d = 64.
 #include <algorithm>
 
 #include "dense.hpp"
@@ -150,15 +156,18 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
 
   f32x4 xk[U], xv[U];  // the next chunk's vectors of this thread
   auto load_chunk = [&](int b, int c0) {
-    const size_t base = (static_cast<size_t>(b) * N + c0) * D;
+    // uniform bases, so a thread's address is a 32-bit offset
+    const size_t base = uniform_offset((static_cast<size_t>(b) * N + c0) * D);
+    const char* const Kb = reinterpret_cast<const char*>(Kx + base);
+    const char* const Vb = reinterpret_cast<const char*>(V + base);
     const int avail = min(kc, N - c0) * VPR;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int v = threadIdx.x + u * bd;
       xk[u] = xv[u] = f32x4{0.f, 0.f, 0.f, 0.f};
       if (v < avail) {
-        xk[u] = *reinterpret_cast<const f32x4*>(Kx + base + 4 * v);
-        xv[u] = *reinterpret_cast<const f32x4*>(V + base + 4 * v);
+        xk[u] = *reinterpret_cast<const f32x4*>(Kb + static_cast<uint32_t>(v) * 16u);
+        xv[u] = *reinterpret_cast<const f32x4*>(Vb + static_cast<uint32_t>(v) * 16u);
       }
     }
   };
@@ -172,9 +181,13 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
   for (int par = 0; blk < nblocks; blk = __builtin_amdgcn_readfirstlane(blk + grid), par ^= 1) {
     const int b = __builtin_amdgcn_readfirstlane(blk / n_qblk), qblk = blk - b * n_qblk;
     const int q0 = __builtin_amdgcn_readfirstlane((qblk * nw + wave) * 32);
-    const size_t boff = static_cast<size_t>(b) * N * D;
+    const size_t boff = uniform_offset(static_cast<size_t>(b) * N * D);
+    // opaque copies of the lane number, here and after the loops: addresses
+    // formed from them are not kept in registers across the loops
+    int pl = lane;
+    asm volatile("" : "+v"(pl));
     RowParts<D> q;
-    q.load(Q + boff + static_cast<size_t>(min(q0 + col, N - 1)) * D, half, scale * kLog2e);
+    q.load(Q + boff + static_cast<size_t>(min(q0 + (pl & 31), N - 1)) * D, pl >> 5, scale * kLog2e);
     f32x16 acc[NB], accl[STACKED ? 1 : NB];  // stacked: elements 8..15 are the lo part's
 #pragma unroll
     for (int n = 0; n < NB; ++n) acc[n] = f32x16{};
@@ -263,8 +276,9 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
             m = max_xor32(m);
             // 2^-x with x = exponent(m) - 5 where m >= 2^11, else 1
             const uint32_t em = __float_as_uint(m) >> 23;
-            const float r = em >= 138u && em < 255u ? __uint_as_float((259u - em) << 23) : 1.f;
-            off -= __builtin_amdgcn_logf(r);
+            const bool up = em >= 138u && em < 255u;
+            const float r = up ? __uint_as_float((259u - em) << 23) : 1.f;
+            off += up ? static_cast<float>(em) - 132.f : 0.f;
             l *= r;
             lb *= r;
 #pragma unroll
@@ -318,18 +332,21 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
       const bool wide = __builtin_amdgcn_readfirstlane(tiny[par]) != 0u;
       const float least = zeros ? 0.f : 1024.f * __builtin_amdgcn_sqrtf(static_cast<float>(N));
       const bool fine = (l >= 16.f) & (a == 0.f) & (big >= least) & (small >= (wide ? l * 0x1p-14f : 0.f));
-      float* const lse_row = lse == nullptr ? nullptr : lse + static_cast<size_t>(b) * 2 * N;
+      int el = lane;
+      asm volatile("" : "+v"(el));
+      const int ecol = el & 31, ehalf = el >> 5;
+      float* const lse_row = lse == nullptr ? nullptr : lse + uniform_offset(static_cast<size_t>(b) * 2 * N);
       if (__any(!fine)) {
 #pragma unroll 1
         for (int t = 0; t < 2; ++t)
           if (q0 + 16 * t < N)
             dense_online_global<D>(Q + boff, Kx + boff, V + boff, O + boff, lse_row, N, q0 + 16 * t,
-                                   lane, scale * kLog2e);
-      } else if (q0 + col < N) {
+                                   el, scale * kLog2e);
+      } else if (q0 + ecol < N) {
         // log2 of the sum by exponent and mantissa: the logarithm's own error
         // is then at the last place of 1, not of log2 l (10 and more)
-        if (lse_row != nullptr && half == 0)
-          lse_row[q0 + col] = (off + static_cast<float>(__builtin_amdgcn_frexp_expf(l))) +
+        if (lse_row != nullptr && ehalf == 0)
+          lse_row[q0 + ecol] = (off + static_cast<float>(__builtin_amdgcn_frexp_expf(l))) +
                               log2f(__builtin_amdgcn_frexp_mantf(l));
         // 1 / vs is a power of two
         const float inv = __builtin_amdgcn_rcpf(l) * __uint_as_float((254u << 23) - __float_as_uint(vs));
@@ -340,7 +357,7 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
             float w[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) w[r] = acc[n][i + r] * inv;
-            st_f32<4>(O + boff + static_cast<size_t>(q0 + col) * D + 32 * n + 2 * i + 4 * half, w);
+            st_f32<4>(O + boff + static_cast<size_t>(q0 + ecol) * D + 32 * n + 2 * i + 4 * ehalf, w);
           }
       }
     }
@@ -372,10 +389,15 @@ static hipError_t launch_dense_split(const DenseArgs& a) {
   while (nw > 4 && a.B * ((waves + nw - 1) / nw) < 2 * kCUs) nw /= 2;  // more CUs at work
   const int n_qblk = (waves + nw - 1) / nw;
   nw = (waves + n_qblk - 1) / n_qblk;
-  if (nw == 8) return launch_dense_split_u<D, 1>(a, nw, n_qblk);
-  // d = 64: two vectors of three waves are less than a 32-key block
-  if (nw >= 4 || D < 64) return launch_dense_split_u<D, 2>(a, nw, n_qblk);
-  return launch_dense_split_u<D, 4>(a, nw, n_qblk);
+  // d = 64: two vectors a thread of fewer than four waves are less than a 32-key
+  // block. Rows of three waves have a fourth that only stages (B=400 N=96: 15.8
+  // -> 14.2 us against four vectors a thread of three), rows of one or two take
+  // four vectors (B=1024 N=40: 14.5 against 19.1 with idle waves).
+  if constexpr (D == 64) {
+    if (nw < 3) return launch_dense_split_u<D, 4>(a, nw, n_qblk);
+    nw = std::max(nw, 4);
+  }
+  return nw == 8 ? launch_dense_split_u<D, 1>(a, nw, n_qblk) : launch_dense_split_u<D, 2>(a, nw, n_qblk);
 }
 
 hipError_t run_dense_split(const DenseArgs& a) {

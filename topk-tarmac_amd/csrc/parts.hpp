@@ -32,6 +32,14 @@ __device__ __forceinline__ float max_xor32(float x) {
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
+// A wave-uniform offset in scalar registers: row offsets computed behind a
+// divergent branch's join are otherwise kept, per lane, in vector registers.
+__device__ __forceinline__ size_t uniform_offset(size_t x) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(x));
+  const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(x >> 32));
+  return static_cast<size_t>(hi) << 32 | lo;
+}
+
 // A barrier that orders LDS accesses only: global loads in flight stay so.
 __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
