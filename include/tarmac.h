@@ -229,8 +229,8 @@ int tarmac_dense_bwd_noalloc(const float* q, const float* k, const float* v, con
  *                   (bf16) cannot change the top k, and exact canonical
  *                   rescoring of the k+1 candidates where it is needed;
  *   packed split -- the packed pass on split-bf16 scores (fp32 inputs,
- *                   d = 16: x = hi + mid + lo, six bf16 products per score),
- *                   proven against the split error bound;
+ *                   d = 16, 32, 64: x = hi + mid + lo, six bf16 products per
+ *                   score), proven against the split error bound;
  *   split32      -- the same on 32-key x 32-query tiles (d = 16, k <= 4,
  *                   N <= 256, bf16 N <= 1024): two lanes per query instead
  *                   of four; bf16
@@ -247,14 +247,14 @@ int tarmac_dense_bwd_noalloc(const float* q, const float* k, const float* v, con
  * sets. The lists path selects on canonical scores and needs no proof.
  * The exactness of the bf16 and split-bf16 proofs rests on a bound for the
  * bf16 MFMA's fp32 accumulation error that is measured, not derived: at most
- * 2^-20.25 of the sum of product magnitudes (worst seen on gfx950: 2^-20.5,
+ * 2^-20.25 of the sum of product magnitudes (worst seen on gfx950: 2^-20.4,
  * one dominant product among small ones; tarmac_mfma_bf16_probe measures
  * it), inside eps = 2^-18 at d <= 32, 2^-17 at d = 64 and 2^-16 at d = 128
  * together with the canonical chain's d 2^-24.
  * mode: 0 = packed always, 1 = automatic (default; the fastest measured on
  * MI355X for the shape), 2 = filter where supported (fp32 d = 16, 32, 64;
  * bf16 d = 16), 3 = lists for fp32 (bf16 runs packed), 4 = packed split where
- * supported (fp32 d = 16; packed elsewhere), 5 = split32 where supported
+ * supported (fp32 d = 16, 32, 64; packed elsewhere), 5 = split32 where supported
  * (d = 16, k <= 4, N <= 256 for fp32 and 1024 for bf16; packed split,
  * then packed, elsewhere). bf16 retained sets are always
  * the exact top k of the canonical fp32 scores of the inputs converted to

@@ -60,7 +60,7 @@ def check_f32(q, k, v, kk, out, idx, exact_order=True):
 def _set_filter(mode: int) -> int:
     """0 = packed pass (fp32 MFMA scores), 1 = automatic, 2 = split-bf16
     filter-and-verify wherever supported, 3 = register-list pass (fp32),
-    4 = packed pass on split-bf16 scores (fp32, d = 16), 5 = the same on
+    4 = packed pass on split-bf16 scores (fp32, d = 16, 32, 64), 5 = the same on
     32 x 32 score tiles (fp32, d = 16, k <= 4, N <= 1024)."""
     from tarmac import _lib
     return _lib.LIB.tarmac_set_topk_filter(mode)

@@ -9,17 +9,19 @@
 namespace tarmac {
 
 // bf16 score error bound, relative to |q| |k_j|: bf16 MFMA sums exact
-// products with an fp32 accumulation error that is measured, not derived
-// (at most 2^-20.25 of the sum of their magnitudes, the worst seen 2^-20.5:
-// one dominant product among small ones, on 16x16x32 and 32x32x16 chains of
-// up to 128 products); the canonical fp32 chain adds <= d 2^-24 of it (one
-// rounding per step); split scores drop three products of <= 2^-24 each;
+// products with an fp32 accumulation error that is measured, not derived: at
+// most 2^-20.25 of the sum of their magnitudes, over 16x16x32 chains of one to
+// four full-size steps (128 products), 32x32x16 chains of six, and the split
+// chains of 3, 6 and 12 steps (d = 16, 32, 64) in their own order and
+// magnitudes; the worst seen is 2^-20.4, one dominant product among small
+// ones. The canonical fp32 chain adds <= d 2^-24 of it (one rounding per
+// step); split scores drop three products of <= 2^-24 each;
 // sum_c |q_c k_c| <= |q| |k_j|. 2^-18 (d <= 32), 2^-17 (d = 64) and 2^-16
 // (d = 128) cover the sum with a margin of 1.25 or more, including the fp32
 // rounding of the bound itself.
 template <int D>
 constexpr float packed_eps() {
-  static_assert(D <= 128, "the bound covers chains of up to 128 products");
+  static_assert(D <= 128, "the bound is measured for widths up to 128");
   return D <= 32 ? 1.0f / 262144.0f : (D <= 64 ? 1.0f / 131072.0f : 1.0f / 65536.0f);
 }
 constexpr float kPackedNormLimit = 1.329228e36f;  // 2^120: |q| max|k| at or above fails the proof
@@ -169,15 +171,21 @@ struct SplitFragWide {
     }
     return f;
   }
+  // The chain's products from the smallest up: three of 2^-16 of the whole,
+  // two of 2^-8, then hi.hi, each over all halves. A bf16 MFMA cuts what it
+  // adds at the accumulator's last place, so only the last D / 32 steps do so
+  // at the score's own magnitude (hi.hi first: 2^-20.0 of sum |q_c k_c| at
+  // d = 64, this order 2^-20.4). mid.mid first keeps the k = 4 kernel at d = 32
+  // within the 128 registers of four waves a SIMD.
   __device__ __forceinline__ f32x4 step(const KF& kf, int i, f32x4 acc) const {
-    const int h = i / 6, p = i % 6;
+    const int p = i / NH, h = i % NH;
     switch (p) {
-      case 0: return mfma_bf16_16x16x32(kf.hi[h], qh[h], acc);
-      case 1: return mfma_bf16_16x16x32(kf.hi[h], qm[h], acc);
-      case 2: return mfma_bf16_16x16x32(kf.mid[h], qh[h], acc);
-      case 3: return mfma_bf16_16x16x32(kf.mid[h], qm[h], acc);
-      case 4: return mfma_bf16_16x16x32(kf.hi[h], ql[h], acc);
-      default: return mfma_bf16_16x16x32(kf.lo[h], qh[h], acc);
+      case 0: return mfma_bf16_16x16x32(kf.mid[h], qm[h], acc);
+      case 1: return mfma_bf16_16x16x32(kf.lo[h], qh[h], acc);
+      case 2: return mfma_bf16_16x16x32(kf.hi[h], ql[h], acc);
+      case 3: return mfma_bf16_16x16x32(kf.mid[h], qh[h], acc);
+      case 4: return mfma_bf16_16x16x32(kf.hi[h], qm[h], acc);
+      default: return mfma_bf16_16x16x32(kf.hi[h], qh[h], acc);
     }
   }
 };
