@@ -92,8 +92,17 @@ def test_one_dominant_coordinate(d, kk, mode):
         check(q, k, v, kk)
 
 
-@pytest.mark.parametrize("B,N,d,kk", [(256, 512, 32, 2), (256, 512, 32, 8), (128, 512, 64, 4),
-                                      (64, 1024, 64, 2)])
+@pytest.mark.parametrize("B,N,d,kk", [(256, 512, 32, 2), (256, 512, 32, 5), (256, 512, 32, 8),
+                                      (256, 1024, 32, 7), (128, 512, 64, 4), (64, 1024, 64, 2),
+                                      (1024, 512, 64, 3), (1024, 704, 64, 3)])
 def test_batches_past_the_line(B, N, d, kk):
-    """Nothing forced: the batch itself takes two query tiles per wave."""
-    check(*qkv(B + N + d, B, N, d), kk)
+    """Nothing forced: the batch itself takes two query tiles per wave, on each
+    side of the lines between the kernels. Sampled rows."""
+    from tarmac.kernels import topk_attention
+    g = torch.Generator().manual_seed(B + N + d + kk)
+    q, k, v = (torch.randn(B, N, d, generator=g) for _ in range(3))
+    out, idx = topk_attention(q.cuda(), k.cuda(), v.cuda(), kk, return_indices=True)
+    rows = [0, 1, B // 2, B - 1]
+    out_c, idx_c = O.canon_topk(*(x[rows].numpy() for x in (q, k, v)), kk)
+    assert np.array_equal(idx[rows].cpu().numpy(), idx_c)
+    assert np.abs(out[rows].cpu().numpy() - out_c).max() <= 1e-5 * np.abs(out_c).max()

@@ -1092,7 +1092,9 @@ enum TopkPath { kPathPacked, kPathPackedSplit, kPathSplit32, kPathFilter, kPathL
 //     6.7 packed, 9.2 split) and the fp32-MFMA packed pass above (N=128 k=4:
 //     17.9 vs 19.9 lists), except at N <= 32, where the one-round-trip list
 //     kernel wins at every k (rocprof, B=1024 N=32 k=4: 7.4 vs 7.8 packed).
-//   fp32, d = 8, 32, 64: register lists for k <= 2 (every k at N <= 32), packed above.
+//   fp32, d = 8, 32, 64: register lists for k <= 2 (every k at N <= 32), packed
+//     above; d = 32 and 64 on rows of 512 keys and more: the packed pass on
+//     split-bf16 scores, the filter or the lists (see choose_path).
 //   bf16: packed, the 32 x 32 kernel at d = 16 with two query tiles per wave
 //     (k = 4, N = 193 .. 256; k = 2, 3, N = 193 .. 384, B <= 1024), or the bf16
 //     filter at d = 16 with N >= 256 and k >= 4
@@ -1167,18 +1169,28 @@ static TopkPath choose_path(const TopkArgs& a, int mode) {
   // at N = 512; at d = 16 the split-bf16 scores stay ahead, N=768: 40.4 vs 47.7)
   if (filt && a.d == 64 && a.topk == 1 && a.N >= 512 && a.N < 1024 && a.B >= 256)
     return kPathFilter;
-  // d = 64, k >= 3 on rows of 512 keys and more from B = 1024: the register
-  // lists (B=1024 N=576 k=8: 800 vs 847 on split-bf16 scores, 860 packed)
-  if (a.d == 64 && a.topk >= 3 && a.N >= 512 && a.B >= 1024) return kPathLists;
+  // d = 64, k >= 3 on rows of 512-703 keys from B = 1024: the register lists
+  // (B=1024 N=512 k=3/4/6: 389/469/533 vs 408/450/528 on split-bf16 scores,
+  // 413/519/586 packed; N=640 572/663/780 vs 611/680/789; B=2048 N=576
+  // 982/1169/1376 vs 1092/1223/1426; from N = 704 the split scores are ahead,
+  // 731/846/997 vs 688/759/893, N=1024 k=4 1597 vs 1249)
+  if (a.d == 64 && a.topk >= 3 && a.N >= 512 && a.N < 704 && a.B >= 1024) return kPathLists;
   // split-bf16 scores at d = 32, 64 (six bf16 products take 6/16 of the fp32
   // MFMA's time, but a split row is 1.4 times an fp32 row in LDS and costs its
   // split): on long rows of batches that take two query tiles per wave. d = 32
-  // from N = 512 (B=256 N=512 k=1/2/4: 38.6/43.0/52.1 vs 43.0 filter, 51.0,
-  // 60.1 packed; B=1024 133.5/147.7/172.3 vs 151.2/179.9/213.0; N=1024
-  // 111/123/145 vs 122/154/199; below, B=1024 N=256 k=2 62.0 vs 53.9 lists).
-  // d = 64 at k >= 3 from N = 512 (B=256 k=4 108.3 vs 121.2 packed), at k = 1, 2 from N = 1024 (B=256
-  // 244.3/264.2 vs 277.4/303.8 lists; N=512 k=2 91.4 vs 90.2).
-  if (split && a.d >= 32 && a.N >= 512 && (a.d == 32 || a.topk >= 3 || a.N >= 1024) &&
+  // from N = 512 (B=256 N=512 k=1/2/4/8: 38.6/43.0/52.1/84.8 vs 43.0 filter,
+  // 51.0, 60.1, 89.7 packed; B=1024 133.5/147.7/172.3/323.7 vs
+  // 151.2/179.9/213.0/335.8; N=1024 111/123/145 vs 122/154/199; below, B=1024
+  // N=256 k=2 62.0 vs 53.9 lists), except at k = 5-7 on rows below 1024 keys from
+  // B = 256, where its registers leave three waves a SIMD (k=5/6/7, B=256 N=512:
+  // 69.1/74.9/88.7 vs 65.8/70.2/74.8 packed; B=1024 264/287/296 vs 231/244/261;
+  // N=768 509/553/564 vs 488/514/549; N=1024 811/878/893 vs 823/863/918).
+  // d = 64 at k >= 3 from N = 512 (B=256 k=4/8: N=512 111/168 vs 123/160 packed,
+  // N=768 197/265 vs 244/303; B=64 to 192 on rows of 512 to 640 keys within 8% of
+  // packed either way), at k = 1, 2 from N = 1024 (B=256 244.3/264.2 vs 277.4/303.8
+  // lists; N=512 k=2 91.4 vs 90.2).
+  const bool split_waves = a.topk <= 4 || a.topk == 8 || a.N >= 1024 || a.B < 256;
+  if (split && a.N >= 512 && ((a.d == 32 && split_waves) || (a.d == 64 && (a.topk >= 3 || a.N >= 1024))) &&
       !one_query_tile(a.B, a.N))
     return kPathPackedSplit;
   // the lists at k <= 2 on rows of up to 128 keys up to B = 256 (B=256

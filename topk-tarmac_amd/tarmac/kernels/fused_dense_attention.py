@@ -23,11 +23,15 @@ def fused_dense_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                           precision: str = "ieee") -> torch.Tensor:
     """Streaming dense self-attention with the diagonal masked. q, k, v: [B, N, d].
 
-    ``precision="ieee"`` is the only fp32 mode: CDNA4's fp32 MFMA is full
-    fp32, and gfx950 has no TF32 path. ``block_kn`` sets the keys staged per
-    LDS pass (rounded up to 16); ``block_m``, ``num_warps`` and ``num_stages``
-    are Triton tiling knobs of the reference and are accepted for signature
-    compatibility only.
+    ``precision="ieee"`` is the only fp32 mode (gfx950 has no TF32 path). It
+    runs on fp32 MFMA, or, at d = 16, 32 and 64 on batches of
+    ``B * ceil(N / 32) >= 1024``, on 16-bit MFMA with every operand split into
+    parts (scores: three bf16 parts, 24 bits; weights and values: two fp16
+    parts, 22 bits; sums in fp32), no further from float64 than fp32 MFMA; rows
+    that parts would not hold run on fp32 MFMA. ``block_kn`` sets the keys
+    staged per LDS pass (rounded up to 16); below N it selects the fp32 MFMA
+    kernel. ``block_m``, ``num_warps`` and ``num_stages`` are Triton tiling
+    knobs of the reference and are accepted for signature compatibility only.
     """
     if precision != "ieee":
         raise ValueError(f"precision={precision!r}: gfx950 has no TF32 mode; use 'ieee'")
