@@ -152,6 +152,24 @@ def test_small_weights_of_large_values(d, log2_value, log2_weight):
     check(fused_dense_attention(q, k, v), exact(q, k, v)[0])
 
 
+@pytest.mark.parametrize("d", [16, 32, 64])
+@pytest.mark.parametrize("N", [128, 256, 1000])
+def test_channels_of_small_weights(N, d):
+    """One-hot values: an output channel is the sum of the weights of the agents
+    it stands for, from 1 down to 2^-20 of the row's largest, and is held to its
+    own size (RTOL: the exponent's rounding, |c s| up to 20 here)."""
+    from tarmac.kernels import fused_dense_attention
+    q, k, v = heads(batch(N), N, d, seed=N)
+    channel = torch.arange(N, device="cuda") % d
+    q[1], k[1] = q[1] * 0.01, k[1] * 0.01
+    q[1, :, 0] = 1.0
+    k[1, :, 0] = channel * (-20.0 / (d - 1) * np.log(2.0) * d ** 0.5)
+    v[1] = torch.nn.functional.one_hot(channel, d).float()
+    out, ref = fused_dense_attention(q, k, v), exact(q, k, v)[0]
+    check(out, ref)
+    assert float(((out[1].double() - ref[1]).abs() / ref[1]).max()) <= RTOL
+
+
 def test_not_finite_stays_in_its_row():
     from tarmac.kernels import fused_dense_attention
     q, k, v = heads(batch(130), 130, 16)

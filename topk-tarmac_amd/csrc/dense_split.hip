@@ -12,11 +12,14 @@
 //       d = 16, where one 32-row operand holds V's hi and lo parts, three of
 //       four above. Three bf16 parts of each (24 bits, no range to see to) cost
 //       21% at d = 16 and gave the same error. V is scaled by a power of two that
-//       puts the row's largest magnitude below 2^15, its lo part by 2^11 more
-//       (its sums are kept apart); P = 2^(c s - off) is kept below 2^15 with a
-//       sum of 2^4 or more.
-//   Error against 64 bits, N(0, 1) inputs, N = 256: 2.1, 2.1, 2.2e-7 at d = 16,
-//   32, 64 (fp32 MFMA: 6.2, 10.4, 4.0e-7); logsumexp 3e-8 off on average (5e-8).
+//       puts the row's largest magnitude below 2^15; P = 2^(c s - off) is kept
+//       below 2^15 with a sum of 2^4 or more. Both lo parts are scaled by 2^11
+//       more, and the products with one of them are summed apart: without that,
+//       weights of 2^-20 of the largest were off by 4e-4 of themselves, which a
+//       channel that only they feed shows (now 1e-6, fp32 MFMA 3e-6), for 5% more
+//       time at d = 16 (B=1024 N=256 30.9 -> 32.5 us; d = 32 and 64 unchanged).
+//   Error against 64 bits, N(0, 1) inputs, N = 256: 1.8, 1.9, 2.0e-7 at d = 16,
+//   32, 64 (fp32 MFMA: 6.1, 10.2, 4.0e-7); logsumexp 3e-8 off on average (5e-8).
 //   The A operand V^T comes from row-major rows by the transposing LDS read.
 //
 // Exponents: off is fixed per query before the first block, the maximum over
@@ -25,21 +28,25 @@
 // at 0 and off is subtracted after: a chain that starts at off is cut at off's
 // magnitude in every product, which the backward sees at scores of 2^5 and more.
 //
-// The result decides whether the parts kept what fp32 keeps: P is held to
-// 2^-25 where it is below 2^-3, scaled V to 2^-36 below 2^-14. A wave with a
-// query whose sum is out of range, whose values are not finite, whose largest
-// channel is small beside what such rounding adds up to, or that has a channel
-// of the size of the smallest parts in a row that holds such elements, runs
-// its queries again on fp32 MFMA with a running maximum, from global memory.
+// The result decides whether the parts kept what fp32 keeps: P and scaled V are
+// held to 2^-36 below 2^-14. A wave with a query whose sum is out of range, whose
+// values are not finite, whose largest channel is small beside what such
+// rounding adds up to, or that has a channel of the size of the smallest parts
+// in a row that holds such elements, runs its queries again on fp32 MFMA with a
+// running maximum, from global memory (B=1024 N=256: one batch row of 1024 adds 20, 48, 73 us at d = 16, 32, 64, all
+// of them take 118, 214, 591; N(0, 1) inputs, also with q 8 times as large and
+// half the values 64 times, meet none).
 //
 // Loads: a workgroup's items (query blocks) and their key chunks form one
 // stream. The next chunk's K and V are loaded into registers while the current
 // one is computed on.
 //
-// Measured against the fp32 MFMA kernel (us): B=1024 N=256 d=16 45.0 -> 31.8,
-// d=32 85.5 -> 47.6, d=64 153 -> 102; B=256 N=1024 d=16 166 -> 100; B=36 N=1000
-// d=64 152 -> 82. About 100 VALU and 10 MFMA per 32 x 32 tile and wave at d = 16,
-// 36 MFMA at d = 64.
+// Measured against the fp32 MFMA kernel (us): B=1024 N=256 d=16 45.0 -> 32.5,
+// d=32 85.5 -> 47.7, d=64 153 -> 103; B=256 N=1024 d=16 166 -> 102; B=36 N=1000
+// d=64 152 -> 81. About 115 VALU and 10 MFMA per 32 x 32 tile and wave at d = 16,
+// 36 MFMA at d = 64. At d = 32 with two vectors a thread 11 lane addresses, each
+// written once and read back once a chunk, do not fit the 128 registers of four
+// waves a SIMD and stay in scratch; the tile loops use none.
 #include <algorithm>
 
 #include "dense.hpp"
@@ -49,7 +56,6 @@ namespace tarmac {
 
 constexpr float kSplitWindow = 5.f;      // log2 of the first tile's largest term
 constexpr float kSplitBlockMax = 0x1p15f;
-constexpr float kLoScale = 0x1p11f;
 
 template <int D>
 struct DenseSplit {
@@ -188,12 +194,11 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
     asm volatile("" : "+v"(pl));
     RowParts<D> q;
     q.load(Q + boff + static_cast<size_t>(min(q0 + (pl & 31), N - 1)) * D, pl >> 5, scale * kLog2e);
-    f32x16 acc[NB], accl[STACKED ? 1 : NB];  // stacked: elements 8..15 are the lo part's
+    // acc: V^T P of the hi parts; accl, scaled by 2^11: hi by lo and lo by hi.
+    // Stacked: acc's elements 8..15 are V's lo by P's hi, accl's are lo by lo.
+    f32x16 acc[NB], accl[NB];
 #pragma unroll
-    for (int n = 0; n < NB; ++n) acc[n] = f32x16{};
-    if constexpr (!STACKED)
-#pragma unroll
-      for (int n = 0; n < NB; ++n) accl[n] = f32x16{};
+    for (int n = 0; n < NB; ++n) acc[n] = accl[n] = f32x16{};
     float off = 0.f, l = 0.f, vs = 0.f;  // vs: the scale of V so far (0: none yet)
     for (int c0 = 0; c0 < N; c0 += kc) {
       const int cn = min(kc, N - c0), kend = c0 + cn;
@@ -239,10 +244,10 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
           const float r = vs == 0.f ? 0.f : vs_new * __uint_as_float((254u << 23) - __float_as_uint(vs));
           vs = vs_new;
 #pragma unroll
-          for (int n = 0; n < NB; ++n) acc[n] *= r;
-          if constexpr (!STACKED)
-#pragma unroll
-            for (int n = 0; n < NB; ++n) accl[n] *= r;
+          for (int n = 0; n < NB; ++n) {
+            acc[n] *= r;
+            accl[n] *= r;
+          }
         }
         for (int kb = 0; kb < cn; kb += 32) {
           f32x16 s = tile_dot<D>(q, Kl + kb * LDK, f32x16{});
@@ -284,10 +289,10 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
 #pragma unroll
             for (int i = 0; i < 16; ++i) e[i] *= r;
 #pragma unroll
-            for (int n = 0; n < NB; ++n) acc[n] *= r;
-            if constexpr (!STACKED)
-#pragma unroll
-              for (int n = 0; n < NB; ++n) accl[n] *= r;
+            for (int n = 0; n < NB; ++n) {
+              acc[n] *= r;
+              accl[n] *= r;
+            }
           }
           l += lb;
 #pragma unroll
@@ -300,9 +305,9 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
 #pragma unroll
             for (int n = 0; n < NB; ++n) {
               const f16x8 vh = __builtin_bit_cast(f16x8, load_t<LDV>(vp + 32 * n));
-              acc[n] = mfma_f16_32(vh, p_lo, acc[n]);
+              accl[n] = mfma_f16_32(vh, p_lo, accl[n]);
               acc[n] = mfma_f16_32(vh, p_hi, acc[n]);
-              if constexpr (!STACKED) 
+              if constexpr (!STACKED)
                 accl[n] = mfma_f16_32(__builtin_bit_cast(f16x8, load_t<LDV>(vp + D + 32 * n)), p_hi, accl[n]);
             }
           }
@@ -316,7 +321,9 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
       for (int n = 0; n < NB; ++n)
 #pragma unroll
         for (int i = 0; i < (STACKED ? 8 : 16); ++i) {
-          acc[n][i] = fmaf(STACKED ? acc[n][(i + 8) % 16] : accl[STACKED ? 0 : n][i], 1.f / kLoScale, acc[n][i]);
+          float lo = accl[n][i];
+          if constexpr (STACKED) lo += fmaf(accl[n][i + 8], 1.f / kLoScale, acc[n][i + 8]);
+          acc[n][i] = fmaf(lo, 1.f / kLoScale, acc[n][i]);
           a = fmaf(0.f, acc[n][i], a);
           big = fmaxf(big, fabsf(acc[n][i]));
           small = fminf(small, fabsf(acc[n][i]));
@@ -324,13 +331,13 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
       big = max_xor32(big);
       // Whether the parts kept what fp32 keeps: the sum of 2^4 or more; every
       // channel finite; the query's largest channel so large that N terms
-      // rounded at 2^-25 beside values below 2^15 stay below 2^-20 of it (a
-      // wave of sharp rows beside values 2^5 and more times theirs fails
+      // rounded at 2^-36 beside values below 2^15 stay below 2^-20 of it (a
+      // wave of sharp rows beside values 2^16 and more times theirs fails
       // this); and, in a row with an element below 2^-14, every channel above
       // 2^-14 of the sum.
       const bool zeros = __builtin_amdgcn_readfirstlane(vmax[par]) == 0u;
       const bool wide = __builtin_amdgcn_readfirstlane(tiny[par]) != 0u;
-      const float least = zeros ? 0.f : 1024.f * __builtin_amdgcn_sqrtf(static_cast<float>(N));
+      const float least = zeros ? 0.f : 0.5f * __builtin_amdgcn_sqrtf(static_cast<float>(N));
       const bool fine = (l >= 16.f) & (a == 0.f) & (big >= least) & (small >= (wide ? l * 0x1p-14f : 0.f));
       int el = lane;
       asm volatile("" : "+v"(el));

@@ -4,7 +4,8 @@
 //
 // Three bf16 parts carry fp32's 24 significand bits and its exponent range;
 // products of 2^-16 of the whole or more are six of nine. Two fp16 parts carry
-// 22 bits of a value whose hi part is normal, in half the instructions.
+// 22 bits of a value whose hi part is normal, in half the instructions; the lo
+// part is kept scaled by 2^11, so that it is normal where hi is.
 #pragma once
 
 #include "frag.hpp"
@@ -15,6 +16,8 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
+
+constexpr float kLoScale = 0x1p11f;  // of the lo part of two fp16 parts
 
 __device__ __forceinline__ f32x16 mfma_bf16_32(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
@@ -76,8 +79,11 @@ __device__ __forceinline__ void split3_dot(float x0, float x1, uint32_t& hi, uin
   lo = __builtin_bit_cast(uint32_t, l);
 }
 
-// Two values as two fp16 pairs: hi rounded to nearest, lo what is left of each
-// (v_fma_mix_f32 subtracts a half of the packed word). 4 VALU a pair.
+// Two values below 2^16 as two fp16 pairs: hi rounded to nearest, lo what is left
+// of it times 2^11, so that a value keeps 22 bits down to 2^-14 and is held to
+// 2^-36 below (unscaled, 2^-25: a weight of 2^-20 beside one of 1 had 10 bits).
+// v_fma_mix_f32 subtracts a half of the packed word; 6 VALU a pair (v_fma_mixlo
+// and mixhi for the last four save one and run no faster).
 __device__ __forceinline__ void split2_pair(float a, float b, uint32_t& hi, uint32_t& lo) {
   const f16x2 h = {static_cast<_Float16>(a), static_cast<_Float16>(b)};
   hi = __builtin_bit_cast(uint32_t, h);
@@ -85,8 +91,8 @@ __device__ __forceinline__ void split2_pair(float a, float b, uint32_t& hi, uint
   const f16x2 hp = __builtin_bit_cast(f16x2, hi);
   float m1;  // -1, opaque: a multiply by a known -1 becomes two conversions and two subtractions
   asm("s_mov_b32 %0, -1.0" : "=s"(m1));
-  const f16x2 l = {static_cast<_Float16>(fmaf(static_cast<float>(hp[0]), m1, a)),
-                   static_cast<_Float16>(fmaf(static_cast<float>(hp[1]), m1, b))};
+  const f16x2 l = {static_cast<_Float16>(fmaf(static_cast<float>(hp[0]), m1, a) * kLoScale),
+                   static_cast<_Float16>(fmaf(static_cast<float>(hp[1]), m1, b) * kLoScale)};
   lo = __builtin_bit_cast(uint32_t, l);
 }
 
