@@ -107,6 +107,24 @@ def test_late_large_scores(d, log2_gap):
 
 
 @pytest.mark.parametrize("d", [16, 32, 64])
+@pytest.mark.parametrize("log2_gap", [120.0, 121.5, 122.2, 122.5, 122.9, 123.5])
+def test_terms_whose_sum_overflows(d, log2_gap):
+    """Two keys of one tile whose terms beside the row's first keys (2^5 there)
+    are near fp32's limit: each still finite, their sum not, from 122 up; from
+    123 each overflows."""
+    from tarmac.kernels import dense_attention_forward_stats
+    q, k, v = heads(batch(200), 200, d)
+    c = np.log2(np.e) / d ** 0.5
+    q[1], k[1, :, 0] = 0.0, 0.0
+    q[1, 17, 0] = 1.0
+    k[1, 70:72, 0] = log2_gap / c
+    out, stats = dense_attention_forward_stats(q, k, v)
+    ref, lse = exact(q, k, v)
+    check(out, ref)
+    assert float((stats[:, 0].double() * np.log(2.0) - lse).abs().max()) <= 2e-5
+
+
+@pytest.mark.parametrize("d", [16, 32, 64])
 @pytest.mark.parametrize("scale", [1e-30, 1e-12, 1e12, 1e30])
 def test_value_scales(d, scale):
     from tarmac.kernels import fused_dense_attention

@@ -285,9 +285,9 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
             const float r = up ? __uint_as_float((259u - em) << 23) : 1.f;
             off += up ? static_cast<float>(em) - 132.f : 0.f;
             l *= r;
-            lb *= r;
+            lb = 0.f;  // summed again: it overflows before the terms do
 #pragma unroll
-            for (int i = 0; i < 16; ++i) e[i] *= r;
+            for (int i = 0; i < 16; ++i) lb += e[i] *= r;
 #pragma unroll
             for (int n = 0; n < NB; ++n) {
               acc[n] *= r;
@@ -329,8 +329,8 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
           small = fminf(small, fabsf(acc[n][i]));
         }
       big = max_xor32(big);
-      // Whether the parts kept what fp32 keeps: the sum of 2^4 or more; every
-      // channel finite; the query's largest channel so large that N terms
+      // Whether the parts kept what fp32 keeps: the sum of 2^4 or more; it and
+      // every channel finite; the query's largest channel so large that N terms
       // rounded at 2^-36 beside values below 2^15 stay below 2^-20 of it (a
       // wave of sharp rows beside values 2^16 and more times theirs fails
       // this); and, in a row with an element below 2^-14, every channel above
@@ -338,7 +338,7 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
       const bool zeros = __builtin_amdgcn_readfirstlane(vmax[par]) == 0u;
       const bool wide = __builtin_amdgcn_readfirstlane(tiny[par]) != 0u;
       const float least = zeros ? 0.f : 0.5f * __builtin_amdgcn_sqrtf(static_cast<float>(N));
-      const bool fine = (l >= 16.f) & (a == 0.f) & (big >= least) & (small >= (wide ? l * 0x1p-14f : 0.f));
+      const bool fine = (l >= 16.f) & (fmaf(0.f, l, a) == 0.f) & (big >= least) & (small >= (wide ? l * 0x1p-14f : 0.f));
       int el = lane;
       asm volatile("" : "+v"(el));
       const int ecol = el & 31, ehalf = el >> 5;
