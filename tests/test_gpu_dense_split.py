@@ -125,6 +125,23 @@ def test_terms_whose_sum_overflows(d, log2_gap):
 
 
 @pytest.mark.parametrize("d", [16, 32, 64])
+@pytest.mark.parametrize("N", [33, 256, 1000])
+@pytest.mark.parametrize("scale", [32, 64, 256])
+def test_sharp_scores(N, d, scale):
+    """Scores so far apart that a tile's terms overflow beside the offset of
+    those before it. The scores' rounding, 2^-24 of the largest |c s| and as
+    much again from the chain, is what a weight is off by."""
+    from tarmac.kernels import fused_dense_attention
+    q, k, v = heads(batch(N), N, d, seed=N + scale)
+    q *= scale
+    s = torch.matmul(q, k.transpose(1, 2).contiguous()) * (np.log2(np.e) / d ** 0.5)
+    out, ref = fused_dense_attention(q, k, v), exact(q, k, v)[0]
+    err = (out.double() - ref).abs().amax(-1) / ref.abs().amax(-1)
+    assert float(err.max()) <= 2.0 ** -23 * float(s.abs().max())
+    assert float((out.double() - ref).norm() / ref.norm()) <= 2.0 ** -25 * float(s.abs().max())
+
+
+@pytest.mark.parametrize("d", [16, 32, 64])
 @pytest.mark.parametrize("scale", [1e-30, 1e-12, 1e12, 1e30])
 def test_value_scales(d, scale):
     from tarmac.kernels import fused_dense_attention

@@ -23,8 +23,12 @@
 //   The A operand V^T comes from row-major rows by the transposing LDS read.
 //
 // Exponents: off is fixed per query before the first block, the maximum over
-// the row's first 32 keys less 5. A block whose terms reach 2^15 raises off by a
-// power of two first (rare: 7 nats above the first keys). Score chains start
+// the row's first 32 keys less 5. A block whose terms add up to 2^15 or more
+// raises off first, which scales by a power of two (rare: 7 nats above the first
+// keys); one whose terms overflow (85 nats above) raises it by 120 and is formed
+// again. With q 32 and 64 times N(0, 1), where many waves meet
+// that, B=1024 N=256 d=16 takes 38 and 40 us (84 and 114 when such waves went to
+// the rerun), d=64 108 and 118 (284 and 589). Score chains start
 // at 0 and off is subtracted after: a chain that starts at off is cut at off's
 // magnitude in every product, which the backward sees at scores of 2^5 and more.
 //
@@ -56,6 +60,7 @@ namespace tarmac {
 
 constexpr float kSplitWindow = 5.f;      // log2 of the first tile's largest term
 constexpr float kSplitBlockMax = 0x1p15f;
+constexpr int kSplitAgain = 32;           // tiles of an item formed again; then the rerun decides
 
 template <int D>
 struct DenseSplit {
@@ -200,6 +205,7 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
 #pragma unroll
     for (int n = 0; n < NB; ++n) acc[n] = accl[n] = f32x16{};
     float off = 0.f, l = 0.f, vs = 0.f;  // vs: the scale of V so far (0: none yet)
+    int again = kSplitAgain;
     for (int c0 = 0; c0 < N; c0 += kc) {
       const int cn = min(kc, N - c0), kend = c0 + cn;
       // V's largest magnitude so far in the row
@@ -274,25 +280,27 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
           for (int i = 0; i < 16; ++i) e[i] = fast_exp2(s[i] - off);
 #pragma unroll
           for (int i = 0; i < 16; ++i) lb += e[i];
-          if (__any(!(lb < kSplitBlockMax))) {  // rare: raise off where a term is out of range
-            float m = 0.f;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) m = fmaxf(m, e[i]);
-            m = max_xor32(m);
-            // 2^-x with x = exponent(m) - 5 where m >= 2^11, else 1
-            const uint32_t em = __float_as_uint(m) >> 23;
-            const bool up = em >= 138u && em < 255u;
-            const float r = up ? __uint_as_float((259u - em) << 23) : 1.f;
-            off += up ? static_cast<float>(em) - 132.f : 0.f;
+          if (__any(!(lb < kSplitBlockMax))) {  // rare: raise off where the sum is out of range
+            // to a sum of 2^9 to 2^10 (a term of 2^5 or more); by 120 where it
+            // overflows, and then the tile is formed again
+            const uint32_t em = __float_as_uint(max_xor32(lb)) >> 23;
+            const uint32_t x = em == 255u ? 120u : em >= 142u ? em - 136u : 0u;
+            const float r = __uint_as_float((127u - x) << 23);
+            off += static_cast<float>(x);
             l *= r;
-            lb = 0.f;  // summed again: it overflows before the terms do
-#pragma unroll
-            for (int i = 0; i < 16; ++i) lb += e[i] *= r;
 #pragma unroll
             for (int n = 0; n < NB; ++n) {
               acc[n] *= r;
               accl[n] *= r;
             }
+            if (__any(em == 255u) && again > 0) {
+              --again;
+              kb -= 32;
+              continue;
+            }
+            lb *= r;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) e[i] *= r;
           }
           l += lb;
 #pragma unroll
