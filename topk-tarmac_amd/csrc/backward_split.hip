@@ -16,9 +16,14 @@
 //     tiles with rows and columns exchanged (lse and D come from LDS);
 //     dV^T += dO^T P, dK^T += Q^T dS.
 //
-// A wave with an output that is not finite, or nonzero and below 2^-80 (parts
+// A column with an output that is not finite, or nonzero and below 2^-80 (parts
 // of its terms may have left their range), runs again on fp32 MFMA from global
-// memory. One barrier a chunk: the next chunk is loaded into registers while
+// memory (B=1024 N=256, every column: 424, 789, 1516 us at d = 16, 32, 64; keys
+// that no one attends to have such gradients where q is 32 times N(0, 1): 145 us
+// at d = 16). Both passes scale the queries and keep the products' order, so
+// they form the bits of the forward's scores and their rounding drops out of
+// s - lse: with pass 2 scaling its keys, dk and dv were 1.4 to 1.6 times as far
+// off as dq with q 16 times N(0, 1) (now 1.0 and 0.9). One barrier a chunk: the next chunk is loaded into registers while
 // the current one is computed on, then split into the other LDS buffer.
 //
 // Measured, both passes, against the fp32 MFMA kernels (us): B=1024 N=256 d=16
@@ -164,7 +169,8 @@ __device__ __forceinline__ void store_grad(float* row, const f32x16 (&acc)[BwdSp
     }
 }
 
-// The rerun of 16 columns on fp32 MFMA from global memory. Columns are queries
+// The rerun of 16 columns on fp32 MFMA from global memory; those whose bit of
+// want is set are stored. Columns are queries
 // (PASS2 false: row matrices A = K, B = V; out_a = dQ) or keys (true: A = Q, B =
 // dO; out_a = dK, out_b = dV). lse, Dq: per query of the batch row.
 template <int D, bool PASS2>
@@ -172,12 +178,12 @@ __device__ __forceinline__ void bwd_rerun(const float* __restrict__ colA, const 
                                           const float* __restrict__ A, const float* __restrict__ Bm,
                                           float lse1, float d1, const float* lse, const float* Dq,
                                           float* __restrict__ out_a, float* __restrict__ out_b, int N,
-                                          int x0, int lane, float scale) {
+                                          int x0, int lane, float scale, uint32_t want) {
   using F = Frag<float, D>;
   constexpr int NH = D / 16;
   const int col = lane & 15, grp = lane >> 4, xi = min(x0 + col, N - 1);
   F fa, fb;
-  fa.load_q(colA + static_cast<size_t>(xi) * D, grp, scale * kLog2eF);
+  fa.load_q(colA + static_cast<size_t>(xi) * D, grp, PASS2 ? 1.f : scale * kLog2eF);
   fb.load_q(colB + static_cast<size_t>(xi) * D, grp, 1.f);
   f32x4 ga[NH], gb[NH];
 #pragma unroll
@@ -185,7 +191,11 @@ __device__ __forceinline__ void bwd_rerun(const float* __restrict__ colA, const 
 #pragma unroll 1
   for (int r0 = 0; r0 < N; r0 += 16) {
     const size_t row = static_cast<size_t>(min(r0 + col, N - 1)) * D;
-    const typename F::KF ka = F::load_k(A + row, grp), kb = F::load_k(Bm + row, grp);
+    typename F::KF ka = F::load_k(A + row, grp);
+    const typename F::KF kb = F::load_k(Bm + row, grp);
+    if constexpr (PASS2)
+#pragma unroll
+      for (int i = 0; i < F::NI; ++i) ka.v[i] *= scale * kLog2eF;
     f32x4 s = {0.f, 0.f, 0.f, 0.f}, dp = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < F::NI; ++i) {
@@ -213,7 +223,7 @@ __device__ __forceinline__ void bwd_rerun(const float* __restrict__ colA, const 
         }
       }
   }
-  if (x0 + col >= N) return;
+  if (x0 + col >= N || (want >> col & 1u) == 0u) return;
 #pragma unroll
   for (int h = 0; h < NH; ++h) {
     float w[4];
@@ -256,6 +266,9 @@ dense_bwd_split_kernel(const float* __restrict__ colA, const float* __restrict__
   const int t_off = piece + upper * 16 + 4 * (lane & 3);  // 16 = D: mid; else the block's next columns
   const int tlo_off = piece + (upper ? 3 * D : 2 * D + 4 * (lane & 3));
 
+  // queries are scaled, in either pass, as in the forward: S - lse is then a
+  // difference of like roundings (see tile_dot)
+  const float c = uniform_value(scale * kLog2eF);
   f32x4 xa[U], xb[U];
   float xs = 0.f, xd = 0.f;
   auto load_chunk = [&](int b, int c0) {
@@ -303,7 +316,7 @@ dense_bwd_split_kernel(const float* __restrict__ colA, const float* __restrict__
     asm volatile("" : "+v"(pl));
     const int xi = min(x0 + (pl & 31), N - 1);
     RowParts<D> pa, pb;
-    pa.load(colA + boff + static_cast<size_t>(xi) * D, pl >> 5, scale * kLog2eF);
+    pa.load(colA + boff + static_cast<size_t>(xi) * D, pl >> 5, PASS2 ? 1.f : c);
     pb.load(colB + boff + static_cast<size_t>(xi) * D, pl >> 5, 1.f);
     float nl = 0.f, nd = 0.f;  // pass 1: -lse and -D of the lane's query
     if constexpr (!PASS2) {
@@ -336,7 +349,7 @@ dense_bwd_split_kernel(const float* __restrict__ colA, const float* __restrict__
       for (int u = 0; u < U; ++u) {
         const int v = threadIdx.x + u * bd, row = v / VPR, cv = v - row * VPR;
         if (row < kc) {
-          store_parts3<D>(As + row * LD + 4 * cv, xa[u]);
+          store_parts3<D>(As + row * LD + 4 * cv, PASS2 ? xa[u] * c : xa[u]);
           store_parts3<D>(Bs + row * LD + 4 * cv, xb[u]);
         }
       }
@@ -353,7 +366,7 @@ dense_bwd_split_kernel(const float* __restrict__ colA, const float* __restrict__
           // the products of each tile before the next tile's scores: P, then
           // dS, is all that is live between them (d = 16 then fits four waves
           // a SIMD; the barriers keep the scheduler from overlapping the two)
-          f32x16 p = tile_dot<D>(pa, As + yb * LD + row_off, f32x16{});
+          f32x16 p = tile_dot<D, PASS2>(pa, As + yb * LD + row_off, f32x16{});
           if constexpr (PASS2) {
 #pragma unroll
             for (int i = 0; i < 16; i += 4) {
@@ -380,7 +393,7 @@ dense_bwd_split_kernel(const float* __restrict__ colA, const float* __restrict__
           for (int i = 0; i < 16; ++i) p[i] = fast_exp2(p[i]);
           if constexpr (PASS2) mma_parts<D>(gb, Bs + yb * LD + t_off, Bs + yb * LD + tlo_off, p);
           __builtin_amdgcn_sched_barrier(0);
-          f32x16 dp = tile_dot<D>(pb, Bs + yb * LD + row_off, f32x16{});
+          f32x16 dp = tile_dot<D, PASS2>(pb, Bs + yb * LD + row_off, f32x16{});
 #pragma unroll
           for (int i = 0; i < 16; i += 4) {
             f32x4 d = {nd, nd, nd, nd};
@@ -400,22 +413,22 @@ dense_bwd_split_kernel(const float* __restrict__ colA, const float* __restrict__
         fold_halves<D>(gb);
         stands &= grad_stands<D>(gb);
       }
-      stands = __all(stands);
+      const uint64_t bad = __ballot(!stands);
+      const uint32_t again = static_cast<uint32_t>(bad) | static_cast<uint32_t>(bad >> 32);
       int el = lane;
       asm volatile("" : "+v"(el));
       const int ecol = el & 31, exi = min(x0 + ecol, N - 1);
-      if (stands) {
-        if (x0 + ecol < N) {
-          store_grad<D>(out_a + boff + static_cast<size_t>(exi) * D, ga, el >> 5, scale);
-          if constexpr (PASS2) store_grad<D>(out_b + boff + static_cast<size_t>(exi) * D, gb, el >> 5, 1.f);
-        }
-      } else {
+      if (x0 + ecol < N && (again >> ecol & 1u) == 0u) {
+        store_grad<D>(out_a + boff + static_cast<size_t>(exi) * D, ga, el >> 5, PASS2 ? uniform_value(scale / c) : scale);
+        if constexpr (PASS2) store_grad<D>(out_b + boff + static_cast<size_t>(exi) * D, gb, el >> 5, 1.f);
+      }
+      if (again != 0u) {
 #pragma unroll 1
         for (int t = 0; t < 2; ++t)
-          if (x0 + 16 * t < N)
+          if (x0 + 16 * t < N && (again >> 16 * t & 0xffffu) != 0u)
             bwd_rerun<D, PASS2>(colA + boff, colB + boff, A + boff, Bm + boff, -__shfl(nl, 16 * t + (el & 15)),
                                 -__shfl(nd, 16 * t + (el & 15)), st, st + N, out_a + boff,
-                                PASS2 ? out_b + boff : nullptr, N, x0 + 16 * t, el, scale);
+                                PASS2 ? out_b + boff : nullptr, N, x0 + 16 * t, el, scale, again >> 16 * t);
       }
     }
   }

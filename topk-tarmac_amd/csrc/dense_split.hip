@@ -26,20 +26,20 @@
 // the row's first 32 keys less 5. A block whose terms add up to 2^15 or more
 // raises off first, which scales by a power of two (rare: 7 nats above the first
 // keys); one whose terms overflow (85 nats above) raises it by 120 and is formed
-// again. With q 32 and 64 times N(0, 1), where many waves meet
-// that, B=1024 N=256 d=16 takes 38 and 40 us (84 and 114 when such waves went to
-// the rerun), d=64 108 and 118 (284 and 589). Score chains start
-// at 0 and off is subtracted after: a chain that starts at off is cut at off's
-// magnitude in every product, which the backward sees at scores of 2^5 and more.
+// again. With q 32 and 64 times N(0, 1), where many waves meet that, B=1024 N=256
+// d=16 takes 36 and 40 us (84 and 114 when such waves went to the rerun), d=64
+// 107 and 118 (284 and 589). Score chains start at 0 and off is subtracted
+// after: a chain that starts at off is cut at off's magnitude in every product,
+// which the backward sees at scores of 2^5 and more.
 //
 // The result decides whether the parts kept what fp32 keeps: P and scaled V are
-// held to 2^-36 below 2^-14. A wave with a query whose sum is out of range, whose
-// values are not finite, whose largest channel is small beside what such
-// rounding adds up to, or that has a channel of the size of the smallest parts
-// in a row that holds such elements, runs its queries again on fp32 MFMA with a
-// running maximum, from global memory (B=1024 N=256: one batch row of 1024 adds 20, 48, 73 us at d = 16, 32, 64, all
-// of them take 118, 214, 591; N(0, 1) inputs, also with q 8 times as large and
-// half the values 64 times, meet none).
+// held to 2^-36 below 2^-14. A query whose sum is out of range, whose values are
+// not finite, whose largest channel is small beside what such rounding adds up
+// to, or that has a channel of the size of the smallest parts in a row that
+// holds such elements, runs again on fp32 MFMA with a running maximum, from
+// global memory (B=1024 N=256: the queries of one batch row of 1024 add 18, 48,
+// 72 us at d = 16, 32, 64, those of all take 114, 214, 578; N(0, 1) inputs, also
+// with q 8 times as large and half the values 64 times, meet none).
 //
 // Loads: a workgroup's items (query blocks) and their key chunks form one
 // stream. The next chunk's K and V are loaded into registers while the current
@@ -48,7 +48,7 @@
 // Measured against the fp32 MFMA kernel (us): B=1024 N=256 d=16 45.0 -> 32.5,
 // d=32 85.5 -> 47.7, d=64 153 -> 103; B=256 N=1024 d=16 166 -> 102; B=36 N=1000
 // d=64 152 -> 81. About 115 VALU and 10 MFMA per 32 x 32 tile and wave at d = 16,
-// 36 MFMA at d = 64. At d = 32 with two vectors a thread 11 lane addresses, each
+// 36 MFMA at d = 64. At d = 32 with two vectors a thread 8 lane addresses, each
 // written once and read back once a chunk, do not fit the 128 registers of four
 // waves a SIMD and stay in scratch; the tile loops use none.
 #include <algorithm>
@@ -76,13 +76,14 @@ struct DenseSplit {
 
 // The rerun: 16 queries of a wave on fp32 MFMA, K and V^T fragments straight
 // from global memory, the running maximum raised per 16-key tile; writes the
-// outputs.
+// outputs of the queries whose bit of want is set.
 template <int D>
 __device__ __forceinline__ void dense_online_global(const float* __restrict__ Qb,
                                                     const float* __restrict__ Kb,
                                                     const float* __restrict__ Vb,
                                                     float* __restrict__ Ob, float* lse, int N,
-                                                    int q0, int lane, float c) {
+                                                    int q0, int lane, float c,
+                                                    uint32_t want) {
   using F = Frag<float, D>;
   constexpr int NH = D / 16;
   const int col = lane & 15, grp = lane >> 4, qi = q0 + col;
@@ -127,7 +128,7 @@ __device__ __forceinline__ void dense_online_global(const float* __restrict__ Qb
       }
   }
   l = add_xor32(add_xor16(l));
-  if (qi >= N) return;
+  if (qi >= N || (want >> col & 1u) == 0u) return;
   if (lse != nullptr && grp == 0) lse[qi] = off + log2f(l);
   const float inv = __builtin_amdgcn_rcpf(l);
 #pragma unroll
@@ -351,13 +352,9 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
       asm volatile("" : "+v"(el));
       const int ecol = el & 31, ehalf = el >> 5;
       float* const lse_row = lse == nullptr ? nullptr : lse + uniform_offset(static_cast<size_t>(b) * 2 * N);
-      if (__any(!fine)) {
-#pragma unroll 1
-        for (int t = 0; t < 2; ++t)
-          if (q0 + 16 * t < N)
-            dense_online_global<D>(Q + boff, Kx + boff, V + boff, O + boff, lse_row, N, q0 + 16 * t,
-                                   el, scale * kLog2e);
-      } else if (q0 + ecol < N) {
+      const uint64_t bad = __ballot(!fine);
+      const uint32_t rerun = static_cast<uint32_t>(bad) | static_cast<uint32_t>(bad >> 32);
+      if (q0 + ecol < N && (rerun >> ecol & 1u) == 0u) {
         // log2 of the sum by exponent and mantissa: the logarithm's own error
         // is then at the last place of 1, not of log2 l (10 and more)
         if (lse_row != nullptr && ehalf == 0)
@@ -374,6 +371,13 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
             for (int r = 0; r < 4; ++r) w[r] = acc[n][i + r] * inv;
             st_f32<4>(O + boff + static_cast<size_t>(q0 + ecol) * D + 32 * n + 2 * i + 4 * ehalf, w);
           }
+      }
+      if (rerun != 0u) {
+#pragma unroll 1
+        for (int t = 0; t < 2; ++t)
+          if (q0 + 16 * t < N && (rerun >> 16 * t & 0xffffu) != 0u)
+            dense_online_global<D>(Q + boff, Kx + boff, V + boff, O + boff, lse_row, N, q0 + 16 * t,
+                                   el, scale * kLog2e, rerun >> 16 * t);
       }
     }
   }

@@ -43,6 +43,11 @@ __device__ __forceinline__ size_t uniform_offset(size_t x) {
   return static_cast<size_t>(hi) << 32 | lo;
 }
 
+// A wave-uniform value in a scalar register.
+__device__ __forceinline__ float uniform_value(float x) {
+  return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x)));
+}
+
 // A barrier that orders LDS accesses only: global loads in flight stay so.
 __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -123,7 +128,9 @@ struct RowParts {
 // parts go in from the smallest up, over all channel groups before the next
 // larger ones, and a chain starts at 0 rather than at a large offset: only the
 // D / 16 products of the hi parts are rounded at the sum's own magnitude.
-template <int D>
+// SWAP: what are columns otherwise are rows here; the products keep their order,
+// so a score has the same bits either way.
+template <int D, bool SWAP = false>
 __device__ __forceinline__ f32x16 tile_dot(const RowParts<D>& q, const bf16* R, f32x16 s) {
   constexpr int G = D / 16;
   // d = 64 reads the rows' hi and mid parts again for the larger products:
@@ -139,15 +146,15 @@ __device__ __forceinline__ f32x16 tile_dot(const RowParts<D>& q, const bf16* R, 
   auto part = [&](int p, int g) { return *(lds_t*)(L + p * D + 16 * g); };
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    s = mfma_bf16_32(part(2, g), q.hi[g], s);
-    s = mfma_bf16_32(part(0, g), q.lo[g], s);
+    s = SWAP ? mfma_bf16_32(part(0, g), q.lo[g], s) : mfma_bf16_32(part(2, g), q.hi[g], s);
+    s = SWAP ? mfma_bf16_32(part(2, g), q.hi[g], s) : mfma_bf16_32(part(0, g), q.lo[g], s);
     s = mfma_bf16_32(part(1, g), q.mid[g], s);
   }
   again();
 #pragma unroll
   for (int g = 0; g < G; ++g) {
-    s = mfma_bf16_32(part(1, g), q.hi[g], s);
-    s = mfma_bf16_32(part(0, g), q.mid[g], s);
+    s = SWAP ? mfma_bf16_32(part(0, g), q.mid[g], s) : mfma_bf16_32(part(1, g), q.hi[g], s);
+    s = SWAP ? mfma_bf16_32(part(1, g), q.hi[g], s) : mfma_bf16_32(part(0, g), q.mid[g], s);
   }
   again();
 #pragma unroll
