@@ -92,6 +92,22 @@ def test_one_dominant_coordinate(d, kk, mode):
         check(q, k, v, kk)
 
 
+@MODES
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("N", [512, 519, 1024, 1300])
+@pytest.mark.parametrize("kk", [1, 2, 3])
+def test_tiles_of_unproven_queries(N, d, kk, mode):
+    """Queries whose keys all tie: a batch row of them, and one with 1, 2, 3 and
+    16 of them to a tile of 16 and in the last tile."""
+    q, k, v = qkv(3 * N + d, 2, N, d)
+    rng = np.random.default_rng(N)
+    q[0], k[0] = (np.eye(d, dtype=np.float32)[rng.integers(0, d, N)] for _ in range(2))
+    for at, n in ((5, 1), (16, 2), (45, 3), (64, 16), (N - 3, 3)):
+        q[1, at:at + n] = 0.0
+    with kernel(mode):
+        check(q, k, v, kk)
+
+
 @pytest.mark.parametrize("B,N,d,kk", [(256, 512, 32, 2), (256, 512, 32, 5), (256, 512, 32, 8),
                                       (256, 1024, 32, 7), (128, 512, 64, 4), (64, 1024, 64, 2),
                                       (1024, 512, 64, 3), (1024, 704, 64, 3)])

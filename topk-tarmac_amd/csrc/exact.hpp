@@ -352,4 +352,50 @@ __device__ __forceinline__ void exact_query_topk_lanes(const T* __restrict__ qro
   }
 }
 
+// The exact top K of 16 queries at once (a query tile, lane l: query q0 + l % 16)
+// for fp32: canonical scores from fp32 MFMA over key rows in global memory, a
+// list of K per lane over its keys, which arrive in ascending order, and a merge
+// of the query's four lanes. A key row is read once for the 16 queries, where the
+// pass above reads it per query, one row a lane; that one is bound by the L1's
+// 64 lines an instruction. Ties make every query of a tile need it: one-hot q and
+// k, B=256 k=2: N=512 d=32 1140 -> 111 us, N=1024 d=64 9050 -> 777.
+template <int D, int K>
+__device__ __forceinline__ void exact_tile_topk(const float* __restrict__ Qb,
+                                                const float* __restrict__ Kb, int N, int q0,
+                                                float scale, int lane, float (&val)[K], int (&ix)[K]) {
+  constexpr bool POW2 = pow2_scale<D>();
+  using F = Frag<float, D>;
+  const int col = lane & 15, grp = lane >> 4;
+  F frag;
+  frag.load_q(Qb + static_cast<size_t>(min(q0 + col, N - 1)) * D, grp, POW2 ? scale : 1.f);
+#pragma unroll
+  for (int m = 0; m < K; ++m) { val[m] = -INFINITY; ix[m] = kIdxSentinel; }
+#pragma unroll 1
+  for (int k0 = 0; k0 < N; k0 += 16) {
+    const typename F::KF kf = F::load_k(Kb + static_cast<size_t>(min(k0 + col, N - 1)) * D, grp);
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < F::NI; ++i) s = frag.step(kf, i, s);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int j = k0 + 4 * grp + r;
+      float x = POW2 ? s[r] : s[r] * scale;
+      if (j >= N || j == q0 + col) x = -INFINITY;
+      topk_insert<K>(val, ix, x, j);
+    }
+  }
+#pragma unroll
+  for (int step = 16; step < 64; step <<= 1) {
+    float pv[K];
+    int pi[K];
+#pragma unroll
+    for (int m = 0; m < K; ++m) {
+      pv[m] = __shfl_xor(val[m], step);
+      pi[m] = __shfl_xor(ix[m], step);
+    }
+#pragma unroll
+    for (int m = 0; m < K; ++m) topk_insert_lex<K>(val, ix, pv[m], pi[m]);
+  }
+}
+
 }  // namespace tarmac

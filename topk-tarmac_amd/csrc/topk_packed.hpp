@@ -39,7 +39,7 @@
 //  5. fallback: an unproven query is recomputed exactly by the whole wave
 //     (exact_query_topk_lanes: its row's canonical scores on the VALU, one
 //     key row per lane, per-lane lists, a six-step merge) -- the result never depends on the packing, only the
-//     time does.
+//     time does. More than a few of them in a tile: see kExactTile.
 //  6. k-softmax and the gathered aggregation over the K value rows.
 //
 // The kernel and its launchers, instantiated per head width by
@@ -58,6 +58,12 @@ namespace tarmac {
 // 16-key tiles per scan block: two keep the block's scores and key fragments
 // at 24 VGPRs (four tiles: 48).
 constexpr int kPackedBlockTiles = 2;
+
+// Unproven queries of a tile above which the tile is recomputed as a whole
+// (split scores at d = 32 and 64, k <= 2, where the choice is between this kernel
+// and the lists, which no tie slows down; at k >= 3 its registers would cost the
+// d = 32 kernel a wave a SIMD).
+constexpr int kExactTile = 2;
 
 // Keys per packing segment for a lane field of FB bits.
 template <int FB>
@@ -475,6 +481,12 @@ topk_packed_kernel(const T* __restrict__ Q, const T* __restrict__ Kx, const T* _
     if (!__all(ok[qt])) {
       // one bit per unproven query (its lane in row 0 stands for it)
       unsigned long long todo = __ballot(grp == 0 && !ok[qt]);
+      if constexpr (SPLIT && D >= 32 && K <= 2) {
+        if (__builtin_popcountll(todo) > kExactTile) {  // the tile's 16 queries at once
+          exact_tile_topk<D, K>(Qb, Kb, N, q0 + 16 * qt, scale, lane, val[qt], ix[qt]);
+          todo = 0ull;
+        }
+      }
       while (todo != 0ull) {
         const int c = __builtin_ctzll(todo);
         todo &= todo - 1ull;
