@@ -95,7 +95,7 @@ def test_one_dominant_coordinate(d, kk, mode):
 @MODES
 @pytest.mark.parametrize("d", [32, 64])
 @pytest.mark.parametrize("N", [512, 519, 1024, 1300])
-@pytest.mark.parametrize("kk", [1, 2, 3])
+@pytest.mark.parametrize("kk", [1, 2, 3, 4, 8])
 def test_tiles_of_unproven_queries(N, d, kk, mode):
     """Queries whose keys all tie: a batch row of them, and one with 1, 2, 3 and
     16 of them to a tile of 16 and in the last tile."""

@@ -59,10 +59,10 @@ namespace tarmac {
 // at 24 VGPRs (four tiles: 48).
 constexpr int kPackedBlockTiles = 2;
 
-// Unproven queries of a tile above which the tile is recomputed as a whole
-// (split scores at d = 32 and 64, k <= 2, where the choice is between this kernel
-// and the lists, which no tie slows down; at k >= 3 its registers would cost the
-// d = 32 kernel a wave a SIMD).
+// Unproven queries of a tile above which the tile is recomputed as a whole, on
+// split scores at d = 64 and at d = 32 with k <= 2: there the choice is between
+// this kernel and the lists, which no tie slows down. (At d = 32 and k >= 3 it is
+// the fp32 packed pass, and the registers would cost a wave a SIMD.)
 constexpr int kExactTile = 2;
 
 // Keys per packing segment for a lane field of FB bits.
@@ -481,7 +481,7 @@ topk_packed_kernel(const T* __restrict__ Q, const T* __restrict__ Kx, const T* _
     if (!__all(ok[qt])) {
       // one bit per unproven query (its lane in row 0 stands for it)
       unsigned long long todo = __ballot(grp == 0 && !ok[qt]);
-      if constexpr (SPLIT && D >= 32 && K <= 2) {
+      if constexpr (SPLIT && (D == 64 || (D == 32 && K <= 2))) {
         if (__builtin_popcountll(todo) > kExactTile) {  // the tile's 16 queries at once
           exact_tile_topk<D, K>(Qb, Kb, N, q0 + 16 * qt, scale, lane, val[qt], ix[qt]);
           todo = 0ull;
