@@ -358,8 +358,8 @@ __device__ __forceinline__ void exact_query_topk_lanes(const T* __restrict__ qro
 // of the query's four lanes. A key row is read once for the 16 queries, where the
 // pass above reads it per query, one row a lane; that one is bound by the L1's
 // 64 lines an instruction. Ties make every query of a tile need it: one-hot q and
-// k, B=256 k=2: N=512 d=32 1140 -> 111 us, N=1024 d=64 9050 -> 777; B=1024 N=1024
-// d=64 k=3 36800 -> 3450.
+// k, B=256 k=2: N=512 d=32 1140 -> 112 us (lists 60), N=1024 d=64 9050 -> 785 (340);
+// B=1024 N=1024 d=64 k=3 36800 -> 3470 (1310).
 template <int D, int K>
 __device__ __forceinline__ void exact_tile_topk(const float* __restrict__ Qb,
                                                 const float* __restrict__ Kb, int N, int q0,

@@ -60,9 +60,8 @@ namespace tarmac {
 constexpr int kPackedBlockTiles = 2;
 
 // Unproven queries of a tile above which the tile is recomputed as a whole, on
-// split scores at d = 64 and at d = 32 with k <= 2: there the choice is between
-// this kernel and the lists, which no tie slows down. (At d = 32 and k >= 3 it is
-// the fp32 packed pass, and the registers would cost a wave a SIMD.)
+// split scores at d = 32 and 64 (whose alternative, the lists, no tie slows down).
+// It comes last and counts its lane numbers again, so it costs no register.
 constexpr int kExactTile = 2;
 
 // Keys per packing segment for a lane field of FB bits.
@@ -473,6 +472,8 @@ topk_packed_kernel(const T* __restrict__ Q, const T* __restrict__ Kx, const T* _
   // exactly at the very end, one at a time across the whole wave, where
   // little else is live, so the rare exact pass does not raise the kernel's
   // register count (and cost waves per SIMD).
+  constexpr bool TILE_PASS = SPLIT && D >= 32;
+  uint32_t tiles = 0u;  // tiles recomputed as a whole, last: one copy, nothing else live
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt)
     if (__all(ok[qt])) finish_tile<T, D, K>(V, O, Idx, b, N, q0 + 16 * qt + col, grp, val[qt], ix[qt]);
@@ -481,10 +482,10 @@ topk_packed_kernel(const T* __restrict__ Q, const T* __restrict__ Kx, const T* _
     if (!__all(ok[qt])) {
       // one bit per unproven query (its lane in row 0 stands for it)
       unsigned long long todo = __ballot(grp == 0 && !ok[qt]);
-      if constexpr (SPLIT && (D == 64 || (D == 32 && K <= 2))) {
-        if (__builtin_popcountll(todo) > kExactTile) {  // the tile's 16 queries at once
-          exact_tile_topk<D, K>(Qb, Kb, N, q0 + 16 * qt, scale, lane, val[qt], ix[qt]);
-          todo = 0ull;
+      if constexpr (TILE_PASS) {
+        if (__builtin_popcountll(todo) > kExactTile) {
+          tiles |= 1u << qt;
+          continue;
         }
       }
       while (todo != 0ull) {
@@ -509,6 +510,18 @@ topk_packed_kernel(const T* __restrict__ Q, const T* __restrict__ Kx, const T* _
         }
       }
       finish_tile<T, D, K>(V, O, Idx, b, N, q0 + 16 * qt + col, grp, val[qt], ix[qt]);
+    }
+  }
+  if constexpr (TILE_PASS) {
+    while (tiles != 0u) {
+      // the lane number counted again: no register is kept for it until here
+      const int tl = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+      const int q1 = q0 + 16 * __builtin_ctz(tiles);
+      tiles &= tiles - 1u;
+      float ev[K];
+      int ei[K];
+      exact_tile_topk<D, K>(Qb, Kb, N, q1, scale, tl, ev, ei);
+      finish_tile<T, D, K>(V, O, Idx, b, N, q1 + (tl & 15), tl >> 4, ev, ei);
     }
   }
 }
