@@ -183,6 +183,18 @@ def profile_one(args, q, k, v, dev) -> int:
             fi()
             fixedset_attention_backward(q7, k7, v7, fi.idx, g7)
             dense_attention_backward(q7, k7, v7, out_d, g7)
+    elif name.startswith("dense_grad"):
+        # a training pass of the dense core at B=1024, N=256: forward with the
+        # logsumexp, and its backward
+        from tarmac.kernels import dense_attention_backward, dense_attention_forward_stats
+        dg = int(name[10:])
+        g = np.random.default_rng(1234 + 7 * 256 + dg)
+        qg, kg, vg, gg = (torch.from_numpy(g.standard_normal((1024, 256, dg)).astype(np.float32))
+                          .to(dev) for _ in range(4))
+
+        def fn():
+            out_g, st_g = dense_attention_forward_stats(qg, kg, vg)
+            dense_attention_backward(qg, kg, vg, out_g, gg, st_g)
     elif name == "dense_small":
         # the memory-bound end of the configs[1] sweep: fp32 dense at B=1024,
         # d=16, N=32 and N=64 (one call of each per step), each beside the
@@ -298,7 +310,8 @@ def main() -> int:
                     help="time only the value kernel (for profiler runs)")
     ap.add_argument("--profile-kernel", default=None,
                     choices=["dense", "dense_bf16", "dense_bf16_d16", "topk1", "topk95", "topk2", "topk4",
-                             "fixedset2", "zorder", "stream2", "large95", "dense_small"],
+                             "fixedset2", "zorder", "stream2", "large95", "dense_small",
+                             "dense_grad16", "dense_grad32", "dense_grad64"],
                     help="run only this kernel (headline shape; zorder/stream at their configs) "
                          "--warmup + --steps times, for profiler counter passes")
     ap.add_argument("--topk-filter", type=int, default=None, choices=[0, 1, 2, 3, 4, 5],

@@ -23,23 +23,27 @@
 // at d = 16). Both passes scale the queries and keep the products' order, so
 // they form the bits of the forward's scores and their rounding drops out of
 // s - lse: with pass 2 scaling its keys, dk and dv were 1.4 to 1.6 times as far
-// off as dq with q 16 times N(0, 1) (now 1.0 and 0.9). One barrier a chunk: the next chunk is loaded into registers while
-// the current one is computed on, then split into the other LDS buffer.
+// off as dq with q 16 times N(0, 1) (now 1.0 and 0.9). One barrier a chunk: the
+// next chunk is loaded into registers while the current one is computed on, then
+// split into the other LDS buffer.
 //
 // Measured, both passes, against the fp32 MFMA kernels (us): B=1024 N=256 d=16
 // 174 -> 120, d=32 298 -> 194, d=64 741 -> 387; B=256 N=512 d=16 165 -> 109;
 // B=300 N=200 d=64 230 -> 113. Per 32 x 32 tile the passes take 20 and 28 MFMA
-// of 33 cycles at d = 16 and 48 and 72 at d = 64, 140 and 240 VALU. Error against
-// 64 bits at d = 16, N = 256: dq, dk, dv 3.3, 3.3, 3.2e-7 (fp32 MFMA 4.7, 4.4,
-// 4.1e-7); N = 512 3.5, 3.4, 3.3e-7 (5.7, 5.2, 5.1e-7); d = 64, N = 256 4.1, 4.1,
-// 4.0e-7 (5.2, 5.2, 4.9e-7).
+// of 33 cycles at d = 16 and 72 and 96 at d = 64, 190 and 300 VALU at d = 16. Bound
+// by issue at d = 16 (traced 51.1 us, VALU 27.1 and MFMA 20.8; pass 2 73.1, 41.0
+// and 28.5), above that (d = 64: 173, 36.1 and 76.1; 219, 47.5 and 102) also by LDS
+// latency at two waves a SIMD. Error against 64 bits at d = 16, N = 256: dq, dk,
+// dv 3.3, 3.3, 3.2e-7 (fp32 MFMA 4.7, 4.4, 4.1e-7); N = 512 3.5, 3.4, 3.3e-7 (5.7,
+// 5.2, 5.1e-7); d = 64, N = 256 4.1, 4.1, 4.0e-7 (5.2, 5.2, 4.9e-7).
 //
 // Registers: at d = 64 pass 2 keeps 96 for its columns' parts and 64 for two
-// accumulators of the 256 that two waves a SIMD leave, and uses no scratch. What
-// else would live across the loops is kept out of it: row offsets are scalars
-// (uniform_offset), and lane addresses outside the loops come from opaque copies
-// of the lane number (with them in registers it spilled 20 to 68, and both
-// passes took B=300 N=200 d=64 133 us).
+// accumulators of the 256 that two waves a SIMD leave, and uses no scratch (pass 1
+// at d = 16 has one register there, read back once a chunk). What else would live
+// across the loops is kept out of it: row offsets are scalars (uniform_offset),
+// and lane addresses outside the loops come from opaque copies of the lane number
+// (with them in registers it spilled 20 to 68, and both passes took B=300 N=200
+// d=64 133 us).
 #include <algorithm>
 
 #include "parts.hpp"

@@ -48,7 +48,9 @@
 // Measured against the fp32 MFMA kernel (us): B=1024 N=256 d=16 45.0 -> 32.5,
 // d=32 85.5 -> 47.7, d=64 153 -> 103; B=256 N=1024 d=16 166 -> 102; B=36 N=1000
 // d=64 152 -> 81. About 115 VALU and 10 MFMA per 32 x 32 tile and wave at d = 16,
-// 36 MFMA at d = 64. At d = 32 with two vectors a thread 8 lane addresses, each
+// 36 MFMA at d = 64. Bound by issue at d = 16 and 32 (B=1024 N=256: VALU 22.9 and
+// MFMA 10.1 of 33.4 us traced, 29.0 and 19.3 of 50.4), at d = 64 (37.9 and 36.6 of
+// 113) also by LDS latency at two waves a SIMD. At d = 32 with two vectors a thread 8 lane addresses, each
 // written once and read back once a chunk, do not fit the 128 registers of four
 // waves a SIMD and stay in scratch; the tile loops use none.
 #include <algorithm>
