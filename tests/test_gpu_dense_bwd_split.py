@@ -77,6 +77,23 @@ def test_sharp_scores(N, d, scale):
 
 
 @pytest.mark.parametrize("d", [16, 32, 64])
+@pytest.mark.parametrize("N", [100, 256, 1000])
+def test_scores_rising_along_the_row(N, d):
+    """Every tile of 32 keys overflows beside the one before it (30 / sqrt(d) nats
+    a key): the forward's logsumexp still comes from the scores that pass 1 forms,
+    so dq, differences of weights next to 1, is as near as on the small-batch
+    kernels (apart: 60 to 200 times as far)."""
+    q, k, v, dout = case(batch(N), N, d, seed=7)
+    k[..., 0] = torch.arange(N, device="cuda") * 30.0
+    q[..., 0] = 1.0
+    n = 2  # rows for which B ceil(N / 32) is below the split kernels' line
+    small = [t[:n].contiguous() for t in (q, k, v, dout)]
+    ref = exact(*small)[0]
+    here, there = grads(q, k, v, dout)[0][:n], grads(*small)[0]
+    assert float((here.double() - ref).norm()) <= 1.5 * float((there.double() - ref).norm())
+
+
+@pytest.mark.parametrize("d", [16, 32, 64])
 def test_launch_shapes(d):
     """Eight-wave workgroups over full rows, more items than workgroups, and
     the logsumexp formed by the backward itself."""

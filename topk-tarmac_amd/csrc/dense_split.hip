@@ -26,7 +26,7 @@
 // the row's first 32 keys less 5. A block whose terms add up to 2^15 or more
 // raises off first, which scales by a power of two (rare: 7 nats above the first
 // keys); one whose terms overflow (85 nats above) raises it by 120 and is formed
-// again. With q 32 and 64 times N(0, 1), where many waves meet that, B=1024 N=256
+// again, up to eight times. With q 32 and 64 times N(0, 1), where many waves meet that, B=1024 N=256
 // d=16 takes 36 and 40 us (84 and 114 when such waves went to the rerun), d=64
 // 107 and 118 (284 and 589). Score chains start at 0 and off is subtracted
 // after: a chain that starts at off is cut at off's magnitude in every product,
@@ -62,7 +62,7 @@ namespace tarmac {
 
 constexpr float kSplitWindow = 5.f;      // log2 of the first tile's largest term
 constexpr float kSplitBlockMax = 0x1p15f;
-constexpr int kSplitAgain = 32;           // tiles of an item formed again; then the rerun decides
+constexpr int kSplitAgain = 8;            // times a tile is formed again; then the rerun decides
 
 template <int D>
 struct DenseSplit {
@@ -286,8 +286,9 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
           if (__any(!(lb < kSplitBlockMax))) {  // rare: raise off where the sum is out of range
             // to a sum of 2^9 to 2^10 (a term of 2^5 or more); by 120 where it
             // overflows, and then the tile is formed again
-            const uint32_t em = __float_as_uint(max_xor32(lb)) >> 23;
-            const uint32_t x = em == 255u ? 120u : em >= 142u ? em - 136u : 0u;
+            const uint32_t mb = __float_as_uint(max_xor32(lb)), em = mb >> 23;
+            const bool over = mb == 0x7f800000u;
+            const uint32_t x = over ? 120u : em >= 142u && em < 255u ? em - 136u : 0u;
             const float r = __uint_as_float((127u - x) << 23);
             off += static_cast<float>(x);
             l *= r;
@@ -296,7 +297,7 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
               acc[n] *= r;
               accl[n] *= r;
             }
-            if (__any(em == 255u) && again > 0) {
+            if (__any(over) && again > 0) {
               --again;
               kb -= 32;
               continue;
@@ -306,6 +307,7 @@ dense_split_kernel(const float* __restrict__ Q, const float* __restrict__ Kx,
             for (int i = 0; i < 16; ++i) e[i] *= r;
           }
           l += lb;
+          again = kSplitAgain;
 #pragma unroll
           for (int t = 0; t < 2; ++t) {
             uint32_t ph[4], pl[4];
