@@ -26,11 +26,11 @@
 // the row's first 32 keys less 5. A block whose terms add up to 2^15 or more
 // raises off first, which scales by a power of two (rare: 7 nats above the first
 // keys); one whose terms overflow (85 nats above) raises it by 120 and is formed
-// again, up to eight times. With q 32 and 64 times N(0, 1), where many waves meet that, B=1024 N=256
-// d=16 takes 36 and 40 us (84 and 114 when such waves went to the rerun), d=64
-// 107 and 118 (284 and 589). Score chains start at 0 and off is subtracted
-// after: a chain that starts at off is cut at off's magnitude in every product,
-// which the backward sees at scores of 2^5 and more.
+// again, up to eight times. With q 32 and 64 times N(0, 1), where many waves meet
+// that, B=1024 N=256 d=16 takes 36 and 40 us (84 and 114 when such waves went to
+// the rerun), d=64 107 and 118 (284 and 589). Score chains start at 0 and off is
+// subtracted after: a chain that starts at off is cut at off's magnitude in every
+// product, which the backward sees at scores of 2^5 and more.
 //
 // The result decides whether the parts kept what fp32 keeps: P and scaled V are
 // held to 2^-36 below 2^-14. A query whose sum is out of range, whose values are
